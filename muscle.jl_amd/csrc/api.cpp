@@ -145,6 +145,59 @@ void plan_gemm_ksplit(Plan& p) {
   }
 }
 
+namespace {
+
+// Whether K's offsets split at multiples of bk: off(k) = off(k - k mod bk) +
+// off(k mod bk) for every k.  They do when a run of bk consecutive k never
+// carries out of a dim: the extents up to some dim divide bk, and that dim's
+// extent is a multiple of what is left (or it is the slowest dim, which only
+// ever counts up).
+bool splits_at(const std::vector<Dim>& k, int64_t bk) {
+  int64_t p = 1;
+  for (size_t i = 0; i < k.size(); ++i) {
+    if (p == bk) return true;
+    if (bk % p) return false;
+    if (p * k[i].extent > bk) return i + 1 == k.size() || k[i].extent % (bk / p) == 0;
+    p *= k[i].extent;
+  }
+  return true;  // at most bk elements in all
+}
+
+// [lo, hi] of the offsets of all points of `v` in operand w
+void offset_range(const std::vector<Dim>& v, int w, int64_t& lo, int64_t& hi) {
+  lo = hi = 0;
+  for (auto& x : v) (x.s[w] < 0 ? lo : hi) += (x.extent - 1) * x.s[w];
+}
+
+// The tile GEMM's per-K-tile addressing (GemmArgs::ktile8): element spans of a
+// K-tile in A and B from the rows' (columns') range and the first 16 k.
+void plan_gemm_ktiles(Plan& p) {
+  const ContractionDesc& d = p.d;
+  if (p.kind != Plan::GEMM) return;
+  int64_t span[2];
+  for (int w = 0; w < 2; ++w) {
+    int64_t lo, hi, klo = 0, khi = 0;
+    offset_range(w == 0 ? d.m : d.n, w, lo, hi);
+    std::vector<Dim> head, rest;
+    int64_t n = 1;
+    for (auto& x : d.k) {
+      if (n >= 16) break;
+      head.push_back(x);
+      head.back().extent = std::min<int64_t>(x.extent, (15 + n) / n);
+      n *= x.extent;
+    }
+    offset_range(head, w, klo, khi);
+    (w == 0 ? p.min_a : p.min_b) = lo + klo;
+    span[w] = (hi + khi - lo - klo + 1) * (int64_t)dtype_size(make_dtype(is_double(d.dt[2]), is_complex(d.dt[w])));
+  }
+  const int64_t lim = int64_t(1) << 32;
+  const bool fits = span[0] < lim && span[1] < lim;
+  p.ktile8 = fits && splits_at(d.k, 8);
+  p.ktile16 = fits && splits_at(d.k, 16);
+}
+
+}  // namespace
+
 // Builds offset tables and picks a kernel for a lowered contraction.
 std::unique_ptr<Plan> build_contraction_plan(const ContractionDesc& d, int precision) {
   std::unique_ptr<Plan> p(new Plan());
@@ -252,6 +305,7 @@ std::unique_ptr<Plan> build_contraction_plan(const ContractionDesc& d, int preci
     p->kind = Plan::REDUCE;
   }
   plan_gemm_ksplit(*p);
+  plan_gemm_ktiles(*p);
   // reduction configuration (also the fallback of the other kinds)
   const int64_t outputs = d.M * d.N * d.B;
   int gshift = 0;
@@ -528,6 +582,10 @@ void run_contraction(Handle& h, Plan& p, const muscle_hip_tensor_t& c, const mus
     g.complex3m = h.complex_mult == 3;
     g.ksplit = q.gemm_ksplit;
     g.kchunk = q.gemm_kchunk;
+    g.ktile8 = q.ktile8;
+    g.ktile16 = q.ktile16;
+    g.minA = q.min_a;
+    g.minB = q.min_b;
     g.partial = base + w.partial_off;
     g.c_stream = csize >= 16 && (double)d.M * (double)d.N * (double)d.B * (double)csize >= kStreamStoreBytes;
     // grid.y carries the batch; split launches beyond the 65535 limit

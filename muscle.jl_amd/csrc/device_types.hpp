@@ -89,7 +89,7 @@ __device__ inline void store_elem_nt(void* base, int64_t off, Cplx<T> v) {
 // fastest, so workgroups running together share A and B panels in their L2.
 __device__ inline void gemm_tile_coords(int L, int nwg, int tiles_m, int tiles_n, int& tm, int& tn) {
   constexpr int GROUP_M = 8;
-  if ((nwg & 7) == 0) L = (L & 7) * (nwg >> 3) + (L >> 3);
+  L = (L & 7) * (nwg >> 3) + min(L & 7, nwg & 7) + (L >> 3);
   const int per_group = GROUP_M * tiles_n;
   const int g = L / per_group;
   const int first_m = g * GROUP_M;

@@ -14,18 +14,42 @@
 //   P1 += ar*br, P2 += ai*bi, P3 += (ar+ai)*(br+bi);
 //   re = P1 - P2, im = P3 - P1 - P2                         (3 MFMAs)
 //
-// Tile: 64 (M) x 64 (N) x BK (K) per 256-thread workgroup, four waves in a
-// 2 x 2 arrangement, each wave a 32 x 32 block of 2 x 2 MFMA 16x16x4 tiles.
-// Operands are staged in LDS as separate real and imaginary planes, double
-// buffered, so one barrier per K-tile suffices.  The global gather of K-tile
-// t+1 and the offset-table reads of K-tile t+2 are in flight while K-tile t
-// is multiplied.  Rows of 64 + 16 elements put the four 16-lane groups of an
-// MFMA operand read in disjoint LDS banks, and the column of element (k, m)
-// is m ^ (k & 15) (a permutation inside each aligned 16-block): the 16 lanes
-// that store 16 consecutive k of one row (operands contiguous along K) then
-// hit 16 different banks instead of one.  Workgroups are renumbered so each
-// XCD (the dispatcher deals workgroups round-robin over 8 XCDs) gets a
-// contiguous, grouped range of tiles and reuses A and B panels in its own L2.
+// One workgroup computes a BM x BN tile of C in K-tiles of BK, its waves
+// arranged WM x WN, each wave a grid of MFMA 16x16x4 tiles.  Operands are
+// staged in LDS as separate real and imaginary planes, double buffered, so one
+// barrier per K-tile suffices; the gather of K-tile t + 1 is in flight while
+// K-tile t is multiplied.
+//
+// What bounds the loop.  A vector instruction does not run beside an FP64 MFMA
+// of the same SIMD: measured on the matrix cores alone, one VALU instruction
+// between two FP64 MFMAs costs 12 cycles of matrix time (an MFMA takes 64), in
+// a run of VALU instructions each further one 2.4 (32-bit) or 4.8 cycles
+// (64-bit and FP64), whatever the number of waves; scalar instructions and LDS
+// reads cost next to nothing.  So the loop keeps vector instructions out:
+//   - a K-tile's elements are addressed from a wave-uniform base (the K offset
+//     of the tile's first k, read through the scalar cache) plus one constant
+//     32-bit register per element, wherever K's offsets split at multiples of
+//     BK (SEP; the host checks it): no address arithmetic is left;
+//   - LDS addresses are constant too (two K-tiles per loop pass, one per
+//     buffer), and the tail of K is a step outside the loop, so no element is
+//     checked inside it;
+//   - the sums ar + ai and br + bi of the 3M form are taken in groups before a
+//     run of MFMAs (scheduling barriers keep the compiler from spreading them).
+// ComplexF64, M = N = K = 4096 on permuted layouts: 7.25 -> 5.64 ms (75.9 ->
+// 97.5 TF, 93 % of the matrix cores' own rate for the 3M products); the loop
+// before waited for each gather in front of its MFMAs and spent 1.8 vector
+// instructions per MFMA.  ComplexF32 64 x 512^3: 574 -> 416 us (120 -> 165 TF).
+// Real FP64 1497 x 1509 x 501: 85 -> 53 us.  Real FP64 4096^3 reaches 69 TF,
+// real FP32 135 TF.  Without a common base per K-tile the ComplexF64 4096 cube
+// takes 6.9 ms, the ComplexF32 case 557 us.
+//
+// Rows of BM + 16 elements put the four 16-lane groups of an MFMA operand read
+// in disjoint LDS banks, and the column of element (k, m) is m ^ swz(k) (a
+// permutation inside each aligned 16-block): the lanes that store consecutive
+// k of one row (operands contiguous along K) then hit different banks.
+// Workgroups are renumbered so each XCD (the dispatcher deals workgroups
+// round-robin over 8 XCDs) gets a contiguous, grouped range of tiles and
+// reuses A and B panels in its own L2.
 //
 // v_mfma_{f64_16x16x4f64, f32_16x16x4f32} lane layout on gfx950 (64 lanes),
 // established with exact small-integer operands on the device:
@@ -33,6 +57,9 @@
 //   B operand: lane l holds B[k = l / 16][j = l % 16]
 //   D (4 regs), f32: lane l, reg r holds D[i = 4 * (l / 16) + r][j = l % 16]
 //   D (4 regs), f64: lane l, reg r holds D[i = l / 16 + 4 * r][j = l % 16]
+#include <algorithm>
+#include <type_traits>
+
 #include "device_types.hpp"
 #include "kernels.hpp"
 
@@ -58,228 +85,389 @@ struct Mfma<float> {
   static __device__ inline int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
-constexpr int BM = 64, BN = 64, NT = 256;
 constexpr int LDP = 16;  // LDS row padding (elements)
 
+// LDS column of row (operand index) m at k: m ^ swz(k), a permutation inside
+// each aligned 16-block.
+template <typename T, int BK>
+__device__ __forceinline__ constexpr int swz(int k) {
+  if (BK == 16) return k & 15;
+  return sizeof(T) == 8 ? (k & 6) << 1 : (k & 4) << 1;
+}
+
+// Entries of one offset table, with one test of its form for all of them.
+template <int N>
+__device__ __forceinline__ void load_offsets(const OffTab& t, const uint32_t* i, int64_t* out) {
+  typedef const MH_GLOBAL int64_t* gp;
+  const gp lo = gptr<int64_t>(t.lo), hi = gptr<int64_t>(t.hi);
+  if (t.single) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] = lo[i[e] + t.base];
+  } else {
+    int64_t h[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const uint32_t x = i[e] + t.base, q = t.div.div(x);
+      out[e] = lo[x - q * t.div.d];
+      h[e] = hi[q];
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] += h[e];
+  }
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MH_CONST __attribute__((address_space(4)))
+#else
+#define MH_CONST
+#endif
+// The entry at a wave-uniform index, read through the scalar cache.
+__device__ __forceinline__ int64_t uniform_offset(const OffTab& t, uint32_t i) {
+  typedef const MH_CONST int64_t* cp;
+  const cp lo = (cp)t.lo, hi = (cp)t.hi;
+  i += t.base;
+  if (t.single) return lo[i];
+  const uint32_t q = t.div.div(i);
+  return lo[i - q * t.div.d] + hi[q];
+}
 
 // T: arithmetic type (MFMA precision); S: storage type of A, B and C.  S = T
 // is the plain path; S = double with T = float is the FP32 rung of the
 // precision ladder (operands rounded to FP32 as they are gathered).
-// MAJ: bit 1 set if A runs contiguous along K (else along M), bit 0 the same
-// for B (else along N), or -1 to read both from the arguments.  Fixed at
-// compile time, the K-offset (or row-offset) registers that every element of
-// a thread shares collapse into one (FP64: 233 -> 227 VGPRs, config 2 from
-// 68 to 70.5 TF; ComplexF32: 160 -> 142..154 VGPRs, config 2 from 128 to
-// 131 TF and the dims-2 4096-cube from 119 to 126 TF).  The FP32 rung of the
-// ladder keeps the run-time form, which measured the same there.
-template <typename T, typename S, bool CA, bool CB, bool G3, int BK, int MAJ>
-__global__ __launch_bounds__(NT, 2) void gemm_tile_kernel(GemmArgs p) {
-  const bool AK = MAJ < 0 ? p.a_kmajor != 0 : (MAJ & 2) != 0;
-  const bool BKM = MAJ < 0 ? p.b_kmajor != 0 : (MAJ & 1) != 0;
+// SEP: the offset of every k is that of its K-tile's first k plus that of its
+// place in the tile, and a tile's elements span less than 2^32 bytes; else
+// K offsets of every K-tile are looked up one K-tile ahead, into LDS.
+// STEPS: MFMA steps (4 k each) whose operands are read and summed together; 0:
+// one at a time, the next step's reads issued ahead of the MFMAs.
+template <typename T, typename S, bool CA, bool CB, bool G3, bool SEP, int BM, int BN, int BK, int WM, int WN, int OCC, int STEPS>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p) {
   using M_ = Mfma<T>;
   using acc_t = typename M_::acc_t;
-  constexpr int NE = BK / 4;  // elements of A (and of B) each thread gathers per K-tile
+  constexpr int NT = 64 * WM * WN;
+  constexpr int NEA = BM * BK / NT, NEB = BN * BK / NT;
   constexpr int PA = CA ? 2 : 1, PB = CB ? 2 : 1;
   constexpr bool CC = CA || CB;
+  constexpr int LA = BM + LDP, LB = BN + LDP;
+  constexpr int TM = BM / WM / 16, TN = BN / WN / 16, KS = BK / 4;
+  constexpr int SA = PA * BK * LA, SB = PB * BK * LB;  // elements of one stage
+  constexpr int64_t EA = sizeof(S) * PA, EB = sizeof(S) * PB;
   static_assert(!G3 || (CA && CB), "3M needs two complex operands");
-  __shared__ T As[2][PA][BK][BM + LDP];
-  __shared__ T Bs[2][PB][BK][BN + LDP];
+  static_assert(NEA >= 1 && NEB >= 1 && BM + BN <= NT, "tile shape");
+  static_assert(2 * (SA + SB) * sizeof(T) >= (BM + BN) * sizeof(int64_t), "C's offsets reuse the stages");
+  __shared__ __attribute__((aligned(16))) T lds[2 * (SA + SB)];  // two A stages, then two B stages
+  __shared__ int64_t koff[SEP ? 1 : 2][2][BK];  // not SEP: byte offsets in A and B of a K-tile's k
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
   int tm, tn;
   gemm_tile_coords(blockIdx.x, gridDim.x, p.tiles_m, p.tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int bz = blockIdx.y;
-  const int64_t offA0 = p.bA[bz], offB0 = p.bB[bz], offC0 = p.bC[bz];
-  // this workgroup's K range (split-K slice)
   const int kbeg = blockIdx.z * p.kchunk;
   const int kend = min(p.K, kbeg + p.kchunk);
+  const int nfull = (kend - kbeg) / BK, tail = (kend - kbeg) % BK;
+  const bool to_partial = p.ksplit > 1;
+  const bool AK = p.a_kmajor != 0, BKM = p.b_kmajor != 0;
 
-  // which (m|n, k) of the tile each thread gathers
-  int a_mm[NE], a_kk[NE], b_nn[NE], b_kk[NE];
+  // this thread's element i of a K-tile: its k, its row (column)
+  auto a_k = [&](int i) { return AK ? tid % BK : tid / BM + NT / BM * i; };
+  auto b_k = [&](int i) { return BKM ? tid % BK : tid / BN + NT / BN * i; };
+  auto a_m = [&](int i) { return AK ? tid / BK + NT / BK * i : tid % BM; };
+  auto b_n = [&](int i) { return BKM ? tid / BK + NT / BK * i : tid % BN; };
+  // Byte offsets in LDS, all constant: the stores of this thread's elements and
+  // this lane's MFMA operand reads at step ks (row k = 4 ks + lane / 16, swizzled
+  // column).  Kept opaque, each stays in a register of its own; buffers and
+  // planes are a multiple of 64 elements apart, so a real and imaginary part
+  // move in one instruction with immediate offsets.
+  uint32_t wa[NEA], wb[NEB], xa[KS][TM], xb[KS][TN];
+  auto opaque = [](uint32_t& v) { asm volatile("" : "+v"(v)); };
 #pragma unroll
-  for (int i = 0; i < NE; ++i) {
-    const int e = tid + NT * i;
-    if (AK) {
-      a_kk[i] = e % BK;
-      a_mm[i] = e / BK;
-    } else {
-      a_mm[i] = e & (BM - 1);
-      a_kk[i] = e >> 6;
+  for (int i = 0; i < NEA; ++i) {
+    wa[i] = (uint32_t)sizeof(T) * (a_k(i) * LA + (a_m(i) ^ swz<T, BK>(a_k(i))));
+    opaque(wa[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NEB; ++i) {
+    wb[i] = (uint32_t)sizeof(T) * (2 * SA + b_k(i) * LB + (b_n(i) ^ swz<T, BK>(b_k(i))));
+    opaque(wb[i]);
+  }
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int kr = ks * 4 + (lane >> 4), c = (lane & 15) ^ swz<T, BK>(kr);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      xa[ks][i] = (uint32_t)sizeof(T) * (kr * LA + c + wm * (BM / WM) + i * 16);
+      opaque(xa[ks][i]);
     }
-    if (BKM) {
-      b_kk[i] = e % BK;
-      b_nn[i] = e / BK;
-    } else {
-      b_nn[i] = e & (BN - 1);
-      b_kk[i] = e >> 6;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      xb[ks][j] = (uint32_t)sizeof(T) * (2 * SA + kr * LB + c + wn * (BN / WN) + j * 16);
+      opaque(xb[ks][j]);
     }
   }
-  int64_t rowA_r[NE], colB_r[NE];
-  bool a_ok[NE], b_ok[NE];
-#pragma unroll
-  for (int i = 0; i < NE; ++i) {
-    const int m = m0 + a_mm[i], n = n0 + b_nn[i];
-    a_ok[i] = m < p.M;
-    b_ok[i] = n < p.N;
-    rowA_r[i] = p.rowA[a_ok[i] ? m : p.M - 1] + offA0;
-    colB_r[i] = p.colB[b_ok[i] ? n : p.N - 1] + offB0;
-    a_mm[i] ^= a_kk[i] & 15;  // from here on: the swizzled LDS columns
-    b_nn[i] ^= b_kk[i] & 15;
-  }
-  const int nk = (kend - kbeg + BK - 1) / BK;
+  auto at = [&](uint32_t off, int e) -> T& { return *((T*)((char*)lds + off) + e); };
 
-  // K-offset table entries of the tile gathered next (indices clamped in range)
-  int64_t tA[NE], tB[NE];
-  auto load_tables = [&](int kt) {
+  // K offsets of K-tile t (the last one's missing k clamped)
+  auto k_offsets = [&](int t, int64_t* ka, int64_t* kb) {
+    const int k0 = kbeg + t * BK, top = (t < nfull ? BK : tail) - 1;
+    uint32_t ia[NEA], ib[NEB];
 #pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      tA[i] = p.kA[min(kbeg + kt * BK + a_kk[i], kend - 1)];
-      tB[i] = p.kB[min(kbeg + kt * BK + b_kk[i], kend - 1)];
+    for (int i = 0; i < NEA; ++i) ia[i] = (uint32_t)(k0 + min(a_k(i), top));
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) ib[i] = (uint32_t)(k0 + min(b_k(i), top));
+    load_offsets<NEA>(p.kA, ia, ka);
+    load_offsets<NEB>(p.kB, ib, kb);
+  };
+  // Rows and columns outside M and N are clamped: they gather valid elements
+  // whose products reach only outputs that are not stored.
+  auto row_offsets = [&](int64_t* om, int64_t* on) {
+    uint32_t im[NEA], in[NEB];
+#pragma unroll
+    for (int i = 0; i < NEA; ++i) im[i] = (uint32_t)min(m0 + a_m(i), p.M - 1);
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) in[i] = (uint32_t)min(n0 + b_n(i), p.N - 1);
+    load_offsets<NEA>(p.rowA, im, om);
+    load_offsets<NEB>(p.colB, in, on);
+  };
+  // not SEP: K-tile t's entry of thread tid < 2 BK (A's k first, then B's)
+  auto k_entry = [&](int t) {
+    const uint32_t i[1] = {(uint32_t)min(kbeg + t * BK + tid % BK, kend - 1)};
+    int64_t o[1];
+    if (tid < BK) load_offsets<1>(p.kA, i, o);
+    else load_offsets<1>(p.kB, i, o);
+    return o[0] * (tid < BK ? EA : EB);
+  };
+  const int64_t offA0 = uniform_offset(p.bA, bz), offB0 = uniform_offset(p.bB, bz), offC0 = uniform_offset(p.bC, bz);
+  Cplx<S> ra[NEA], rb[NEB];
+  auto zero_tail = [&]() {  // both operands beyond K
+#pragma unroll
+    for (int i = 0; i < NEA; ++i)
+      if (a_k(i) >= tail) ra[i] = Cplx<S>{S(0), S(0)};
+#pragma unroll
+    for (int i = 0; i < NEB; ++i)
+      if (b_k(i) >= tail) rb[i] = Cplx<S>{S(0), S(0)};
+  };
+  const int nk = nfull + (tail ? 1 : 0);
+  uint32_t va[NEA], vb[NEB];      // SEP: byte offsets inside a K-tile
+  const char *pa[NEA], *pb[NEB];  // else: row (column) addresses
+  const char* const bA = (const char*)p.A + (offA0 + p.minA) * EA;
+  const char* const bB = (const char*)p.B + (offB0 + p.minB) * EB;
+  {
+    int64_t om[NEA], on[NEB], ka[NEA], kb[NEB];
+    row_offsets(om, on);
+    k_offsets(0, ka, kb);
+#pragma unroll
+    for (int i = 0; i < NEA; ++i) ra[i] = load_elem<S, CA>(p.A, offA0 + om[i] + ka[i]);
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) rb[i] = load_elem<S, CB>(p.B, offB0 + on[i] + kb[i]);
+    if constexpr (SEP) {
+      const int64_t a0 = uniform_offset(p.kA, kbeg) + p.minA, b0 = uniform_offset(p.kB, kbeg) + p.minB;
+#pragma unroll
+      for (int i = 0; i < NEA; ++i) va[i] = (uint32_t)((om[i] + ka[i] - a0) * EA);
+#pragma unroll
+      for (int i = 0; i < NEB; ++i) vb[i] = (uint32_t)((on[i] + kb[i] - b0) * EB);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NEA; ++i) pa[i] = (const char*)p.A + (offA0 + om[i]) * EA;
+#pragma unroll
+      for (int i = 0; i < NEB; ++i) pb[i] = (const char*)p.B + (offB0 + on[i]) * EB;
+      if (tid < 2 * BK && nk > 1) koff[1][tid / BK][tid % BK] = k_entry(1);
+    }
+    if (nfull == 0) zero_tail();
+  }
+  auto gather = [&](int t) {  // whole K-tile t (SEP), or any
+    if constexpr (SEP) {
+      const char* ga = bA + uniform_offset(p.kA, kbeg + t * BK) * EA;
+      const char* gb = bB + uniform_offset(p.kB, kbeg + t * BK) * EB;
+#pragma unroll
+      for (int i = 0; i < NEA; ++i) {
+        asm volatile("" : "+v"(va[i]));  // keeps the 32-bit offset a register of its own
+        ra[i] = load_elem<S, CA>(ga + va[i], 0);
+      }
+#pragma unroll
+      for (int i = 0; i < NEB; ++i) {
+        asm volatile("" : "+v"(vb[i]));
+        rb[i] = load_elem<S, CB>(gb + vb[i], 0);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NEA; ++i) ra[i] = load_elem<S, CA>(pa[i] + koff[t & 1][0][a_k(i)], 0);
+#pragma unroll
+      for (int i = 0; i < NEB; ++i) rb[i] = load_elem<S, CB>(pb[i] + koff[t & 1][1][b_k(i)], 0);
     }
   };
-  Cplx<T> ra[NE], rb[NE];
-  // a tile whose rows and columns all lie inside M and N needs no per-element
-  // checks on the K-tiles that lie inside its K range (all but the last);
-  // FP64 data on FP32 MFMA keeps the checked form, which measured faster there
-  const bool full_mn = sizeof(T) == sizeof(S) && m0 + BM <= p.M && n0 + BN <= p.N;
-  auto gather = [&](int kt) {
-    if (full_mn && kbeg + (kt + 1) * BK <= kend) {
+  auto gather_tail = [&]() {  // the last K-tile, of fewer than BK k
+    if constexpr (SEP) {
+      int64_t om[NEA], on[NEB], ka[NEA], kb[NEB];
+      row_offsets(om, on);
+      k_offsets(nfull, ka, kb);
 #pragma unroll
-      for (int i = 0; i < NE; ++i) {
-        const Cplx<S> xa = load_elem<S, CA>(p.A, rowA_r[i] + tA[i]);
-        const Cplx<S> xb = load_elem<S, CB>(p.B, colB_r[i] + tB[i]);
-        ra[i] = Cplx<T>{(T)xa.re, (T)xa.im};
-        rb[i] = Cplx<T>{(T)xb.re, (T)xb.im};
-      }
-      return;
-    }
+      for (int i = 0; i < NEA; ++i) ra[i] = load_elem<S, CA>(p.A, offA0 + om[i] + ka[i]);
 #pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      const Cplx<S> xa = load_elem<S, CA>(p.A, rowA_r[i] + tA[i]);
-      const Cplx<S> xb = load_elem<S, CB>(p.B, colB_r[i] + tB[i]);
-      ra[i] = Cplx<T>{(T)xa.re, (T)xa.im};
-      rb[i] = Cplx<T>{(T)xb.re, (T)xb.im};
-      const bool ka = kbeg + kt * BK + a_kk[i] < kend, kb = kbeg + kt * BK + b_kk[i] < kend;
-      if (!(a_ok[i] && ka)) ra[i] = Cplx<T>{T(0), T(0)};
-      if (!(b_ok[i] && kb)) rb[i] = Cplx<T>{T(0), T(0)};
+      for (int i = 0; i < NEB; ++i) rb[i] = load_elem<S, CB>(p.B, offB0 + on[i] + kb[i]);
+    } else {
+      gather(nfull);
     }
   };
   auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      // a_mm / b_nn hold the swizzled LDS columns by now
-      As[buf][0][a_kk[i]][a_mm[i]] = ra[i].re;
-      if constexpr (CA) As[buf][PA - 1][a_kk[i]][a_mm[i]] = ra[i].im;
-      Bs[buf][0][b_kk[i]][b_nn[i]] = rb[i].re;
-      if constexpr (CB) Bs[buf][PB - 1][b_kk[i]][b_nn[i]] = rb[i].im;
+    for (int i = 0; i < NEA; ++i) {
+      at(wa[i], buf * SA) = (T)ra[i].re;
+      if constexpr (CA) at(wa[i], buf * SA + BK * LA) = (T)ra[i].im;
+    }
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) {
+      at(wb[i], buf * SB) = (T)rb[i].re;
+      if constexpr (CB) at(wb[i], buf * SB + BK * LB) = (T)rb[i].im;
     }
   };
 
-  acc_t acc0[2][2], acc1[2][2], acc2[2][2];
+  acc_t acc0[TM][TN], acc1[TM][TN], acc2[TM][TN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        acc0[i][j][r] = T(0);
-        acc1[i][j][r] = T(0);
-        acc2[i][j][r] = T(0);
-      }
-
-  load_tables(0);
-  gather(0);
-  stash(0);
-  if (nk > 1) load_tables(1);
-  __syncthreads();
-
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) gather(kt + 1);
-    if (kt + 2 < nk) load_tables(kt + 2);
-    // FP64: the MFMA section issues at raised wave priority, so a wave that is
-    // multiplying is not held back by the other workgroup's waves issuing
-    // their gathers and LDS stores (config 2: 71.1 -> 76.2 TF)
-    if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
+      for (int r = 0; r < 4; ++r) acc0[i][j][r] = acc1[i][j][r] = acc2[i][j][r] = T(0);
+  struct Frag {
+    T ar[TM], ai[TM], as[TM], br[TN], bi[TN], bs[TN];
+  };
+  auto read_frag = [&](int buf, int ks, Frag& f) {
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = ks * 4 + (lane >> 4);
-      T ar[2], ai[2], br[2], bi[2];
+    for (int i = 0; i < TM; ++i) {
+      f.ar[i] = at(xa[ks][i], buf * SA);
+      f.ai[i] = CA ? at(xa[ks][i], buf * SA + BK * LA) : T(0);
+    }
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int mm = (wm * 32 + i * 16 + (lane & 15)) ^ (kr & 15);
-        ar[i] = As[cur][0][kr][mm];
-        ai[i] = CA ? As[cur][PA - 1][kr][mm] : T(0);
-        const int nn = (wn * 32 + i * 16 + (lane & 15)) ^ (kr & 15);
-        br[i] = Bs[cur][0][kr][nn];
-        bi[i] = CB ? Bs[cur][PB - 1][kr][nn] : T(0);
-      }
-      if constexpr (G3) {
-        T as[2], bs[2];
+    for (int j = 0; j < TN; ++j) {
+      f.br[j] = at(xb[ks][j], buf * SB);
+      f.bi[j] = CB ? at(xb[ks][j], buf * SB + BK * LB) : T(0);
+    }
+  };
+  auto sums = [&](Frag& f) {
+    if constexpr (G3) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          as[i] = ar[i] + ai[i];
-          bs[i] = br[i] + bi[i];
+      for (int i = 0; i < TM; ++i) f.as[i] = f.ar[i] + f.ai[i];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) f.bs[j] = f.br[j] + f.bi[j];
+    } else if constexpr (CA && CB) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) f.as[i] = -f.ai[i];
+    }
+  };
+  auto multiply = [&](const Frag& f) {
+    if constexpr (G3) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          acc0[i][j] = M_::mma(f.ar[i], f.br[j], acc0[i][j]);
+          acc1[i][j] = M_::mma(f.ai[i], f.bi[j], acc1[i][j]);
+          acc2[i][j] = M_::mma(f.as[i], f.bs[j], acc2[i][j]);
+        }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          acc0[i][j] = M_::mma(f.ar[i], f.br[j], acc0[i][j]);
+          if constexpr (CB) acc1[i][j] = M_::mma(f.ar[i], f.bi[j], acc1[i][j]);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            acc0[i][j] = M_::mma(ar[i], br[j], acc0[i][j]);
-            acc1[i][j] = M_::mma(ai[i], bi[j], acc1[i][j]);
-            acc2[i][j] = M_::mma(as[i], bs[j], acc2[i][j]);
-          }
-      } else {
-        // acc0: real part, acc1: imaginary part
+        for (int j = 0; j < TN; ++j) {
+          if constexpr (CA && CB) acc0[i][j] = M_::mma(f.as[i], f.bi[j], acc0[i][j]);
+          if constexpr (CA) acc1[i][j] = M_::mma(f.ai[i], f.br[j], acc1[i][j]);
+        }
+    }
+  };
+
+  stash(0);
+  __syncthreads();
+  // K-tile t from LDS buffer cur; inner steps have a whole K-tile after theirs
+  auto step = [&](int t, auto cur_, auto inner_) {
+    constexpr int cur = decltype(cur_)::value;
+    constexpr bool inner = decltype(inner_)::value;
+    if (inner || t + 1 < nfull) gather(t + 1);
+    else if (t + 1 < nk) gather_tail();
+    int64_t kn = 0;  // K-tile t + 2's offsets replace K-tile t's
+    if constexpr (!SEP)
+      if (tid < 2 * BK && t + 2 < nk) kn = k_entry(t + 2);
+    if constexpr (STEPS == 0) {
+      // step by step, the next step's reads ahead of this step's MFMAs
+      Frag f[2];
+      read_frag(cur, 0, f[0]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int ks = 0; ks < KS; ++ks) {
+        sums(f[ks & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ks + 1 < KS) read_frag(cur, ks + 1, f[(ks + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f[ks & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      Frag f[STEPS];
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            acc0[i][j] = M_::mma(ar[i], br[j], acc0[i][j]);
-            if constexpr (CA && CB) acc0[i][j] = M_::mma(-ai[i], bi[j], acc0[i][j]);
-            if constexpr (CB) acc1[i][j] = M_::mma(ar[i], bi[j], acc1[i][j]);
-            if constexpr (CA) acc1[i][j] = M_::mma(ai[i], br[j], acc1[i][j]);
-          }
+      for (int k0 = 0; k0 < KS; k0 += STEPS) {
+#pragma unroll
+        for (int e = 0; e < STEPS; ++e) read_frag(cur, k0 + e, f[e]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < STEPS; ++e) sums(f[e]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < STEPS; ++e) multiply(f[e]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(0);
-    if (kt + 1 < nk) stash(cur ^ 1);
-    __syncthreads();
-  }
-
-  // partial sums of a split-K slice go to the workspace, [split][batch][m][n]
-  const bool to_partial = p.ksplit > 1;
-  const int64_t pbase = ((int64_t)blockIdx.z * gridDim.y + bz) * (int64_t)p.M * p.N;
-  // C's offsets for this thread's rows and columns, read before any store
-  // (a table load after a store to C could not be hoisted: they may alias)
-  int64_t crow[2][4], ccol[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm * 32 + i * 16 + M_::row(lane, r);
-      crow[i][r] = (!to_partial && m < p.M) ? p.rowC[m] : 0;
+    if (inner || t + 1 < nk) {
+      if (!inner && t + 1 == nfull) zero_tail();
+      stash(cur ^ 1);
+      if constexpr (!SEP)
+        if (tid < 2 * BK && t + 2 < nk) koff[cur][tid / BK][tid % BK] = kn;
     }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int n = n0 + wn * 32 + j * 16 + (lane & 15);
-    ccol[j] = n < p.N ? (to_partial ? pbase + n : offC0 + p.colC[n]) : 0;
+    __syncthreads();
+  };
+  constexpr std::integral_constant<int, 0> B0;
+  constexpr std::integral_constant<int, 1> B1;
+  constexpr std::true_type inner;
+  constexpr std::false_type ending;
+  int t = 0;
+  for (; t + 2 < nfull; t += 2) {
+    step(t, B0, inner);
+    step(t + 1, B1, inner);
   }
+  step(t, B0, ending);
+  if (t + 1 < nk) step(t + 1, B1, ending);
+  if (t + 2 < nk) step(t + 2, B0, ending);
+
+  // C's offsets, one lookup per thread, through the stages' LDS
+  int64_t* coff = reinterpret_cast<int64_t*>(lds);
+  if (!to_partial && tid < BM + BN) {
+    const uint32_t i[1] = {(uint32_t)(tid < BM ? min(m0 + tid, p.M - 1) : min(n0 + tid - BM, p.N - 1))};
+    int64_t o[1];
+    if (tid < BM) load_offsets<1>(p.rowC, i, o);
+    else load_offsets<1>(p.colC, i, o);
+    coff[tid] = o[0];
+  }
+  __syncthreads();
+  // partial sums of a split-K slice go to the workspace, [split][batch][m][n]
+  const int64_t pbase = ((int64_t)blockIdx.z * gridDim.y + bz) * (int64_t)p.M * p.N;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < TN; ++j) {
+    const int nl = wn * (BN / WN) + j * 16 + (lane & 15);
+    if (n0 + nl >= p.N) continue;
+    const int64_t cn = to_partial ? pbase + n0 + nl : offC0 + coff[BM + nl];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn * 32 + j * 16 + (lane & 15);
-      if (n >= p.N) continue;
-      const int64_t cn = ccol[j];
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm * 32 + i * 16 + M_::row(lane, r);
-        if (m >= p.M) continue;
+        const int ml = wm * (BM / WM) + i * 16 + M_::row(lane, r);
+        if (m0 + ml >= p.M) continue;
         T re, im;
         if constexpr (G3) {
           re = acc0[i][j][r] - acc1[i][j][r];
@@ -288,13 +476,13 @@ __global__ __launch_bounds__(NT, 2) void gemm_tile_kernel(GemmArgs p) {
           re = acc0[i][j][r];
           im = acc1[i][j][r];
         }
-        if (to_partial) store_elem<T, CC>(p.partial, cn + (int64_t)m * p.N, Cplx<T>{re, im});
-        else if (p.c_stream) store_elem_nt<S, CC>(p.C, cn + crow[i][r], Cplx<S>{(S)re, (S)im});
-        else store_elem<S, CC>(p.C, cn + crow[i][r], Cplx<S>{(S)re, (S)im});
+        if (to_partial) store_elem<T, CC>(p.partial, cn + (int64_t)(m0 + ml) * p.N, Cplx<T>{re, im});
+        else if (p.c_stream) store_elem_nt<S, CC>(p.C, cn + coff[ml], Cplx<S>{(S)re, (S)im});
+        else store_elem<S, CC>(p.C, cn + coff[ml], Cplx<S>{(S)re, (S)im});
       }
     }
+  }
 }
-
 // C[bz, m, n] = sum over slices s of partial[s][bz][m][n], in slice order.
 // Small (64-thread) workgroups spread the few outputs of a split-K GEMM over
 // many CUs, and the unrolled slice loop keeps 8 loads of each thread in flight.
@@ -318,18 +506,67 @@ __global__ __launch_bounds__(NTF) void splitk_finish_kernel(GemmArgs p) {
   store_elem<S, CC>(p.C, p.bC[bz] + p.rowC[m] + p.colC[n], Cplx<S>{(S)re, (S)im});
 }
 
+// A tile configuration of gemm_tile_kernel.
+template <int BM_, int BN_, int BK_, int WM_, int WN_, int OCC_, int STEPS_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, OCC = OCC_, STEPS = STEPS_;
+  // complex FP64 64x64x16 fills the LDS of two workgroups per CU: no room for the K offset table
+  static constexpr bool SEP_ONLY = BM == 64 && BN == 64 && BK == 16 && OCC == 2;
+};
+
+template <typename T, typename S, bool CA, bool CB, bool G3, typename C>
+void launch_tile(GemmArgs g, hipStream_t s) {
+  g.tiles_m = (g.M + C::BM - 1) / C::BM;
+  g.tiles_n = (g.N + C::BN - 1) / C::BN;
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)g.batch, (unsigned)g.ksplit), block(64 * C::WM * C::WN);
+  if (C::BK == 8 ? g.ktile8 : g.ktile16)
+    hipLaunchKernelGGL(
+        (gemm_tile_kernel<T, S, CA, CB, G3, true, C::BM, C::BN, C::BK, C::WM, C::WN, C::OCC, C::STEPS>), grid, block, 0,
+        s, g);
+  else if constexpr (C::SEP_ONLY)
+    ;  // chosen for its K-tiles' common base only
+  else
+    hipLaunchKernelGGL(
+        (gemm_tile_kernel<T, S, CA, CB, G3, false, C::BM, C::BN, C::BK, C::WM, C::WN, C::OCC, C::STEPS>), grid, block,
+        0, s, g);
+}
+
+// Tile shapes by the number of 64 x 64 tiles (and K slices) of the launch.
+// Large tiles read the least; where there are too few of them to spread evenly
+// over the workgroups that fit 256 CUs, smaller tiles win, and in complex FP64
+// also where K is so short that a tile spends its time in its first loads and
+// its stores.  Measured (us; N x N x 512 unless noted, tiles of 64 x 64 first):
+//   complex FP64, 64x64x8 / 32x64x8 / 32x32x8: N = 1024: 80 / 66 / 58, 1536:
+//     143 / 129 / 122, 2048: 231 / 203 / 213, 4096: 729 / 766 / 795;
+//     4096 x 4096 with K = 8 / 32 / 128: 52 / 82 / 209 against 47 / 82 / 219
+//     for 32x64x8; K = 4096: 5.69 ms, 5.59 with 64x64x16 (78 KB more LDS, two
+//     workgroups per CU in place of three, half the barriers);
+//   real FP64, 64x64x16 / 32x32x16: 1024: 32 / 26, 1536: 58 / 52, 2048: 75 / 88;
+//   ComplexF32, 64x64x8 / 32x64x16: 1024: 46 / 34, 1536: 75 / 76, 2048: 101 / 110;
+//   real FP32, 64x64x16 / 32x64x16: 1024: 22 / 17, 1536: 35 / 30, 2048: 43 / 49.
 template <typename T, typename S, bool CA, bool CB, bool G3>
 void launch_t(const GemmArgs& g, hipStream_t s) {
-  dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)g.batch, (unsigned)g.ksplit);
-  if constexpr (sizeof(T) != sizeof(S)) {
-    hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, 16, -1>), grid, dim3(NT), 0, s, g);
-  } else {
-    switch ((g.a_kmajor ? 2 : 0) | (g.b_kmajor ? 1 : 0)) {
-      case 0: hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, 16, 0>), grid, dim3(NT), 0, s, g); break;
-      case 1: hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, 16, 1>), grid, dim3(NT), 0, s, g); break;
-      case 2: hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, 16, 2>), grid, dim3(NT), 0, s, g); break;
-      default: hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, 16, 3>), grid, dim3(NT), 0, s, g); break;
+  const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch * g.ksplit;
+  const int k = std::min(g.K, g.kchunk);
+  if constexpr (sizeof(T) == 8 && CA && CB) {
+    if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 8, 2, 2, 6, 1>>(g, s);
+    else if (tiles < 2048 || k <= 32) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 1>>(g, s);
+    else if (G3 && k >= 1024 && g.ktile16) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 2, 2>>(g, s);
+    else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, G3 ? 3 : 2, 1>>(g, s);
+  } else if constexpr (sizeof(T) == 8) {
+    if constexpr (CA || CB) {
+      if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 2>>(g, s);
+      else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, 3, 1>>(g, s);
+    } else {
+      if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 16, 2, 2, 6, 4>>(g, s);
+      else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 4, 1>>(g, s);
     }
+  } else if constexpr (CA || CB) {
+    if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
+    else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, sizeof(S) == 8 ? 3 : 4, 1>>(g, s);
+  } else {
+    if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
+    else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, sizeof(S) == 8 ? 3 : 4, 4>>(g, s);
   }
   if (g.ksplit > 1) {
     const int64_t total = (int64_t)g.M * g.N * g.batch;
@@ -342,8 +579,6 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
 
 void launch_gemm_mfma(bool dbl, bool fp32_math, bool ca, bool cb, const GemmArgs& g0, hipStream_t s) {
   GemmArgs g = g0;
-  g.tiles_m = (g.M + BM - 1) / BM;
-  g.tiles_n = (g.N + BN - 1) / BN;
   if (g.ksplit < 1) {
     g.ksplit = 1;
     g.kchunk = g.K;

@@ -42,6 +42,9 @@ struct Plan {
   }
   bool a_kmajor = false, b_kmajor = false;
   bool fp32_math = false;  // FP64 operands multiplied on FP32 MFMA (precision FP32)
+  // K-tiles of 8 / 16 addressed from one base per tile (GemmArgs::ktile8)
+  bool ktile8 = false, ktile16 = false;
+  int64_t min_a = 0, min_b = 0;
   // tile GEMM split-K
   int gemm_ksplit = 1;
   int gemm_kchunk = 0;

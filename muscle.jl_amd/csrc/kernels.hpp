@@ -77,6 +77,12 @@ struct GemmArgs {
   int32_t ksplit, kchunk;
   void* partial;
   int32_t c_stream;  // store C with nontemporal (streaming) stores
+  // K-tiles of 8 (16) k are addressed from one base per tile: off(k) of A and B
+  // is off(k - k mod 8) + off(k mod 8), and the elements of a tile span less
+  // than 2^32 bytes above offsets minA and minB (of the rows or columns and the
+  // first 16 k together)
+  int32_t ktile8, ktile16;
+  int64_t minA, minB;
 };
 // Complex FP64 outputs of at least this many bytes are written with
 // nontemporal stores: they do not stay in the caches anyway (writing C bounds

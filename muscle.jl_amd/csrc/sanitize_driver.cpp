@@ -4,7 +4,8 @@
 // be preloaded into another process.
 //
 //   sanitize_driver          lowering and argument checking through
-//                            muscle_hip_describe (no GPU needed)
+//                            muscle_hip_describe, and the tile GEMM's K-tile
+//                            addressing against its offset tables (no GPU needed)
 //   sanitize_driver --gpu    additionally: random contractions, a batch in all
 //                            three run modes and a server with contraction-tree
 //                            jobs, each against a naive host loop over every
@@ -20,9 +21,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <random>
 #include <vector>
 
+#include "handle.hpp"
 #include "muscle_hip.h"
 
 namespace {
@@ -207,6 +210,62 @@ std::vector<cd> random_values(const Operand& o, std::mt19937_64& rng) {
 }
 
 size_t esize(int dt) { return dt == MUSCLE_HIP_F32 ? 4 : dt == MUSCLE_HIP_F64 ? 8 : dt == MUSCLE_HIP_C32 ? 8 : 16; }
+// A plan's K-tile addressing (ktile8, ktile16, min_a, min_b) against its offset
+// tables: where a flag is set, off(k) = off(k - k mod bk) + off(k mod bk) for
+// every k of both operands, and the elements of a K-tile lie in [min, min +
+// 2^32 bytes).
+void check_ktiles(std::mt19937_64& rng) {
+  int64_t set = 0, plans = 0;
+  for (int it = 0; it < 3000; ++it) {
+    const int nk = 1 + (int)(rng() % 4);
+    std::vector<int64_t> extent(1, 1);
+    std::vector<int32_t> lk, la, lb, lc;
+    for (int i = 0; i < nk; ++i) {
+      const int64_t choices[] = {2, 2, 3, 4, 5, 8, 9, 16, 24, 33};
+      extent.push_back(choices[rng() % 10]);
+      lk.push_back((int32_t)extent.size() - 1);
+    }
+    extent.push_back(32 + (int64_t)(rng() % 40));
+    la = lk;
+    la.push_back((int32_t)extent.size() - 1);
+    lc.push_back((int32_t)extent.size() - 1);
+    extent.push_back(32 + (int64_t)(rng() % 40));
+    lb = lk;
+    lb.push_back((int32_t)extent.size() - 1);
+    lc.push_back((int32_t)extent.size() - 1);
+    Operand a = make_operand(la, extent, rng), b = make_operand(lb, extent, rng), c = make_operand(lc, extent, rng);
+    for (auto& st : a.strides)
+      if (rng() % 8 == 0) st = -st;  // reversed modes
+    for (auto& st : b.strides)
+      if (rng() % 64 == 0) st <<= 26;  // spans past 2^32 bytes
+    const muscle_hip_tensor_t tc = c.desc(MUSCLE_HIP_F64, (void*)256), ta = a.desc(MUSCLE_HIP_F64, (void*)256),
+                              tb = b.desc(MUSCLE_HIP_F64, (void*)256);
+    const std::unique_ptr<mh::Plan> p =
+        mh::build_contraction_plan(mh::lower_binary(tc, ta, tb), MUSCLE_HIP_PRECISION_NATIVE);
+    if (p->kind != mh::Plan::GEMM) continue;
+    ++plans;
+    for (int64_t bk : {8, 16}) {
+      bool splits = true, fits = true;
+      for (int w = 0; w < 2; ++w) {
+        const std::vector<int64_t> k = mh::offset_table(p->d.k, w), r = mh::offset_table(w == 0 ? p->d.m : p->d.n, w);
+        for (size_t i = 0; i < k.size(); ++i)
+          splits = splits && k[i] == k[i - i % (size_t)bk] + k[i % (size_t)bk];
+        const int64_t lo = *std::min_element(r.begin(), r.end()), hi = *std::max_element(r.begin(), r.end());
+        const size_t n = std::min<size_t>(k.size(), 16);
+        const int64_t klo = *std::min_element(k.begin(), k.begin() + n), khi = *std::max_element(k.begin(), k.begin() + n);
+        const int64_t base = w == 0 ? p->min_a : p->min_b;
+        expect(base <= lo + klo, "K-tile base above an element", it);
+        fits = fits && (hi + khi - base + 1) * 8 < (int64_t(1) << 32);
+      }
+      const bool flag = bk == 8 ? p->ktile8 : p->ktile16;
+      expect(!flag || (splits && fits), "K-tile addressing of offsets that do not split or fit", it);
+      set += flag;
+    }
+  }
+  expect(set > plans / 2, "most plans have a common base per K-tile", set);
+  std::printf("%lld tile GEMM plans checked, %lld K-tile sizes with a common base\n", (long long)plans, (long long)set);
+}
+
 bool is_cplx(int dt) { return dt == MUSCLE_HIP_C32 || dt == MUSCLE_HIP_C64; }
 
 std::vector<char> encode(const std::vector<cd>& v, int dt) {
@@ -457,6 +516,8 @@ void check_gpu(std::mt19937_64& rng) {
 int main(int argc, char** argv) {
   std::mt19937_64 rng(20261203);
   check_describe(rng);
+  std::mt19937_64 rng_k(20261204);
+  check_ktiles(rng_k);
   if (argc > 1 && std::strcmp(argv[1], "--gpu") == 0) check_gpu(rng);
   std::printf("%s: %d failures\n", g_failures ? "FAILED" : "ok", g_failures);
   return g_failures ? 1 : 0;
