@@ -108,7 +108,7 @@ typedef struct {
 
 /* What the library did for one contraction (optional out-parameter). */
 typedef struct {
-  int32_t kernel;        /* 0 none, 1 MFMA tile GEMM, 2 reduction, 3 split-precision, 4 elementwise,
+  int32_t kernel;        /* 0 none, 1 MFMA tile GEMM, 2 reduction and power-of-two (vector FMA), 3 split-precision, 4 elementwise,
                             5 (unused),
                             6 tiled permutation (unary_einsum with no summed modes, transposed through LDS),
                             7 Ozaki int8 in modular form: int8 MFMA products modulo small moduli,

@@ -196,6 +196,26 @@ void plan_gemm_ktiles(Plan& p) {
   p.ktile16 = fits && splits_at(d.k, 16);
 }
 
+// The contraction runs in its operands' own precision (no ladder rung).
+bool precision_plain(const ContractionDesc& d, int precision) {
+  return precision == MUSCLE_HIP_PRECISION_NATIVE || !is_double(d.dt[2]) || d.M < 16 || d.N < 16 || d.K < 16;
+}
+
+// Contractions the power-of-two kernel is for, by what the other kernels
+// measured on the same pairs (complex FP64, us, other / power-of-two).  A sum
+// too short for the matrix tiles: 2^2 x 2^20 x 2^2 145 / 25, 2^12 x 2^12 x 2 167
+// / 61, but 2^8 x 2^8 x 2 x 2 (64 tiles) 4.2 / 4.7: from 128 tiles on.  Both
+// sides 32 or more: K = 8, 2^6 x 2^6 8.1 / 5.2, 2^12 x 2^12 85 / 57; K = 16,
+// 2^12 x 2^12 86 / 77, with kept modes 2^16 x 2^6 (x 4) 90 / 96: only without
+// them.  A short side and K = 16 to 128: 2^4 x 2^18 x 2^6 184 / 98, 2^3 x 2^18 x
+// 2^7 307 / 242, 2^4 x 2^14 x 2^6 x 2 (256 tiles) 25 / 39, K = 256 from 1.7
+// times faster to 1.3 times slower: from 512 tiles and up to K = 128.
+bool bits_wanted(const ContractionDesc& d) {
+  const double tiles = (double)d.M * (double)d.N * (double)d.B / (1 << kBitTile);
+  if (std::min(d.M, d.N) >= 32) return d.K < 8 ? tiles >= 128 : d.K == 8 || (d.K == 16 && d.B == 1);
+  return d.K <= 8 ? tiles >= 128 : std::min(d.M, d.N) <= 16 && d.K <= 128 && tiles >= 512;
+}
+
 }  // namespace
 
 // Builds offset tables and picks a kernel for a lowered contraction.
@@ -205,6 +225,12 @@ std::unique_ptr<Plan> build_contraction_plan(const ContractionDesc& d, int preci
   p->precision = precision;
   if (d.empty) {
     p->kind = Plan::EMPTY;
+    return p;
+  }
+  // Little work per output and power-of-two extents throughout: tiles of C in
+  // address order.
+  if (d.has_b && precision_plain(d, precision) && bits_wanted(d) && plan_bits(d, p->bits)) {
+    p->kind = Plan::BITS;
     return p;
   }
   const int64_t lim32 = int64_t(1) << 32;
@@ -439,7 +465,7 @@ void fill_info(muscle_hip_info_t* info, const Plan& p, const muscle_hip_tensor_t
   std::memset(info, 0, sizeof *info);
   const ContractionDesc& d = p.d;
   info->kernel = p.kind == Plan::GEMM      ? 1
-                 : p.kind == Plan::REDUCE  ? 2
+                 : p.kind == Plan::REDUCE || p.kind == Plan::BITS ? 2
                  : p.kind == Plan::SPLIT   ? (p.split_mode == kSplitModeCrt ? (p.crt_split ? 8 : 7) : 3)
                  : p.kind == Plan::PERMUTE ? 6
                                            : 0;
@@ -531,6 +557,15 @@ void run_contraction(Handle& h, Plan& p, const muscle_hip_tensor_t& c, const mus
   int dta, dtb = d.dt[1];
   const void* A = promote_operand(h, *ka, dbl, cursor, dta);
   const void* B = kb ? promote_operand(h, *kb, dbl, cursor, dtb) : nullptr;
+  if (p.kind == Plan::BITS) {
+    BitDesc b = p.bits;
+    b.L = p.bits.long_b ? B : A;
+    b.S = p.bits.long_b ? A : B;
+    b.C = c.data;
+    launch_bits_one(dbl, is_complex(d.dt[2]), b, h.stream);
+    check_launch();
+    return;
+  }
   if (p.kind == Plan::SPLIT) {
     run_split(h, p, c.data, A, B, is_complex(dta), is_complex(dtb), base + w.split_off);
     check_launch();
@@ -641,7 +676,7 @@ std::unique_ptr<Plan> make_plan(Handle& h, int kind, int precision, double targe
   std::unique_ptr<Plan> np = build_contraction_plan(d, precision);
   if (np->kind == Plan::SPLIT) prepare_split(*np, target);
   consider_packing(*np);
-  if (np->kind != Plan::EMPTY) upload_tables(*np, h.stream);
+  if (np->kind != Plan::EMPTY && np->kind != Plan::BITS) upload_tables(*np, h.stream);
   if (np->inner) upload_tables(*np->inner, h.stream);
   upload_split_tables(*np, h.stream);
   return np;
@@ -911,15 +946,16 @@ int muscle_hip_binary_einsum_noalloc(muscle_hip_handle_t handle, const muscle_hi
     // cached device allocation, and operands are gathered where they lie
     // (no packed copies)
     std::unique_ptr<Plan> p = build_contraction_plan(lower_binary(*c, *a, *b), MUSCLE_HIP_PRECISION_NATIVE);
-    if (p->kind != Plan::EMPTY && p->kind != Plan::GEMM && p->kind != Plan::REDUCE)
+    if (p->kind != Plan::EMPTY && p->kind != Plan::GEMM && p->kind != Plan::REDUCE && p->kind != Plan::BITS)
       fail(MUSCLE_HIP_UNSUPPORTED, "binary_einsum_noalloc: unsupported contraction plan");
-    const size_t tab = p->kind == Plan::EMPTY ? 0 : align_up(p->htab.size() * sizeof(int64_t));
+    const bool tables = p->kind != Plan::EMPTY && p->kind != Plan::BITS;
+    const size_t tab = !tables ? 0 : align_up(p->htab.size() * sizeof(int64_t));
     const size_t need = tab + contraction_workspace_bytes(*p, *a, b);
     if (need > kScratchBytes)
       fail(MUSCLE_HIP_INVALID_ARGUMENT, "binary_einsum_noalloc: this contraction needs " + std::to_string(need) +
                                             " bytes of scratch (offset tables, partial sums, casts); the maximum is " +
                                             std::to_string(kScratchBytes));
-    if (p->kind != Plan::EMPTY) {
+    if (tables) {
       // stream-ordered after the previous call's kernels, which may still read the old tables
       MH_HIP_CHECK(hipMemcpyAsync(h->scratch, p->htab.data(), p->htab.size() * sizeof(int64_t),
                                   hipMemcpyHostToDevice, h->stream));

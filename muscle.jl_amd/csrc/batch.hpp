@@ -144,7 +144,15 @@ struct Batch {
   std::vector<int2> hitems;
   int32_t qoff[kXcds + 1] = {0};  // the persistent items' per-XCD queues (offsets into hitems)
   int32_t nq = 1;                 // queues in use (kXcds or 1)
-  int64_t nskinny = 0;   // the skinny items at the end of hitems
+  // shallow and skinny pairs of power-of-two extents run in the power-of-two
+  // kernel: their items (descriptor, first tile) at the end of hitems, their
+  // descriptors, the largest LDS need, each pair's descriptor (-1: none)
+  int64_t nbits = 0;
+  int bits_lds = 0;
+  std::vector<BitDesc> hbits;
+  std::vector<int32_t> bit_index;
+  BitDesc* dbits = nullptr;
+  int64_t nskinny = 0;   // the skinny items before them
   int64_t nshallow = 0;  // the shallow items before them
   // of them, those of pairs with C along N, along M, then the same two with
   // streaming stores for C
@@ -157,6 +165,9 @@ struct Batch {
   int64_t ntilecnt = 0;
   size_t partial_bytes = 0;
   int64_t split_items = 0;
+  // tiles of the shallow pairs, items of the skinny ones and all items as
+  // reported (by the routes' own tile sizes, whichever kernel runs a pair)
+  int64_t shallow_tiles = 0, skinny_tiles = 0, all_tiles = 0;
   bool allow_split = true;  // off for the autotuner's timing batches
   std::vector<int64_t> htab;
   std::vector<int> pair_class;
@@ -190,8 +201,8 @@ constexpr double kBatchSoloPoints = double(int64_t(1) << 29);
 
 // Location of one two-level table inside a batch's table arena.
 struct TabRef {
-  size_t lo, hi;
-  uint32_t P, single;
+  size_t lo = 0, hi = 0;
+  uint32_t P = 1, single = 1;
 };
 
 // One pair after host planning.
@@ -207,13 +218,17 @@ struct PlannedPair {
   const int64_t* dtab = nullptr;  // device tables of this pair; null: the batch's own table region
   const std::vector<int64_t>* htab = nullptr;  // the host copy its TabRefs index
   bool solo = false;              // runs as a single-contraction launch, not in the work list
+  // bits: the power-of-two kernel takes the pair in any launch where its route
+  // is shallow or skinny; bits_only: it has no other route, and no tables
+  bool bits = false, bits_only = false;
+  BitDesc bit;
 };
 
-// Device layout of a planned batch: pairs | items | counter | tables, copied
+// Device layout of a planned batch: pairs | items | bits | counter | tables, copied
 // from the host (the first `copy` bytes), then the split pairs' arrival
 // counters and partial tiles, device-only.
 struct BatchLayout {
-  size_t pairs, items, counter, tab, tilecnt, partial, copy, total;
+  size_t pairs, items, bits, counter, tab, tilecnt, partial, copy, total;
 };
 // A pair of at most kSplitMaxTiles output tiles and at least kSplitMinKTiles
 // K-tiles (16 K each) runs as K slices (split kernel).
@@ -232,6 +247,9 @@ void plan_pair(const Handle& h, PlannedPair& L, std::vector<int64_t>& htab, int 
 // points on, which keeps the tables (host time and upload) small at one more
 // lookup per index.
 constexpr int64_t kTickSingleMax = 256;
+// The power-of-two kernel's pairs (bits_pair; those of other extents keep the
+// shallow and skinny kernels).
+constexpr int64_t kBitMinTiles = 256, kBitSkinnyMaxK = 128, kBitSkinnyMinTiles = 512;
 // Work list (the persistent items, largest K first, then the shallow pairs'
 // items), workgroup count and LDS size of the pairs in lw.
 void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw);

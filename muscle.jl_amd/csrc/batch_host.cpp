@@ -87,6 +87,21 @@ void copy_desc(Batch& b, const muscle_hip_tensor_t& t, std::vector<muscle_hip_te
   dst.push_back(t);
 }
 
+// Shallow or skinny pairs that the power-of-two kernel is for (complex FP64, us):
+// the 256 pairs of a circuit network to rank 22, all by the other two kernels
+// 5213, by this one 4138, and 4215 where pairs of fewer than 128 of its tiles
+// stay with them (a launch of their own).  Where every pair is small they stay:
+// a server's ticks (up to 64 tiles a pair) ran this kernel for 52 us, of which
+// most is fetching its code and descriptors once, the others for 12 and 20.
+// A longer K is a chain of gathers: 2^3 x 2^8 x 2^7 (x 4) on its 4 tiles took
+// 60 us longer than the skinny kernel when its operands were in HBM, so from
+// 512 tiles on, as for a single contraction.
+bool bits_pair(const ContractionDesc& d, bool others) {
+  const double tiles = (double)d.M * (double)d.N * (double)d.B / (1 << kBitTile);
+  if (d.K <= kShallowK) return others || tiles >= kBitMinTiles;
+  return std::min(d.M, d.N) <= kSkinnyMaxS && d.K <= kBitSkinnyMaxK && tiles >= kBitSkinnyMinTiles;
+}
+
 }  // namespace
 
 int batch_tuning_class(int64_t m, int64_t n) { return tuning_class(m, n); }
@@ -117,8 +132,10 @@ void plan_pair(const Handle& h, PlannedPair& L, std::vector<int64_t>& htab, int 
   const int64_t lim = int64_t(1) << 31;
   if (d.M >= lim || d.N >= lim || d.K >= lim || d.B >= lim)
     fail(MUSCLE_HIP_UNSUPPORTED, "batched pair with an index class of 2^31 or more elements");
+  L.bits = bits_pair(d, false) && plan_bits(d, L.bit);
+  L.bits_only = L.bits && d.K <= kShallowK;
   const std::vector<Dim>* cls[4] = {&d.m, &d.n, &d.k, &d.batch};
-  for (int t = 0; t < 9; ++t) L.t[t] = add_table(htab, *cls[T3[t][0]], T3[t][1], single_max);
+  for (int t = 0; t < 9 && !L.bits_only; ++t) L.t[t] = add_table(htab, *cls[T3[t][0]], T3[t][1], single_max);
   L.htab = &htab;
   if (tile < 0 || tile >= MUSCLE_HIP_TILE_COUNT) {
     const int tc = h.tune[tuning_class(d.M, d.N)];
@@ -180,7 +197,14 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
     q.k = L.d.K;
     q.batch = L.d.B;
   }
-  std::vector<int2> shallow[4], sliced, skinny, xq[kXcds], single;
+  std::vector<int2> shallow[4], sliced, skinny, bits, xq[kXcds], single;
+  B.bit_index.assign((size_t)n, -1);
+  B.bits_lds = 0;
+  B.shallow_tiles = B.skinny_tiles = 0;
+  B.hbits.clear();
+  const bool run_bits =
+      std::any_of(lw.begin(), lw.end(), [](const PlannedPair* L) { return L->bits && !L->solo; });
+  BitDesc small;
   double xload[kXcds] = {0, 0, 0, 0, 0, 0, 0, 0};
   const int sko = skinny_outputs(is_double(B.dtype), cp);
   for (int64_t i : order) {
@@ -246,6 +270,13 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
         for (int64_t t = 0; t < items; ++t) xq[x].push_back(make_int2((int)i, (int)t));
         xload[x] += cost * (double)items;
       }
+    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small)))) {
+      const int32_t x = (int32_t)B.hbits.size();
+      B.bit_index[(size_t)i] = x;
+      B.hbits.push_back(L.bits ? L.bit : small);
+      const BitDesc& q = B.hbits.back();
+      for (int32_t t = 0; t < q.tiles; t += q.run) bits.push_back(make_int2(x, t));
+      B.bits_lds = std::max(B.bits_lds, q.nl + q.ns);
     } else if (sh || sk) {
       // the vector-FMA kernels are bound by writing C: their items go in the
       // order of their corners' addresses in C, so the tiles that run at the
@@ -279,6 +310,8 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
       for (int64_t t = 0; t < items * ks; ++t) sliced.push_back(make_int2((int)i, (int)t));
     }
     if (!sh && !sk) used[L.tile] = true;
+    if (sk) B.skinny_tiles += items;
+    else if (sh) B.shallow_tiles += items;
   }
   size_t nq = 0;
   for (int x = 0; x < kXcds; ++x) nq += xq[x].size();
@@ -305,6 +338,9 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
   }
   B.nskinny = (int64_t)skinny.size();
   B.hitems.insert(B.hitems.end(), skinny.begin(), skinny.end());
+  B.nbits = (int64_t)bits.size();
+  B.all_tiles = (int64_t)nq + B.nsplit + B.shallow_tiles + B.skinny_tiles;
+  B.hitems.insert(B.hitems.end(), bits.begin(), bits.end());
   const bool dbl = is_double(B.dtype);
   for (int t = 0; t < MUSCLE_HIP_TILE_COUNT; ++t)
     if (used[t]) B.lds = std::max(B.lds, batch_lds_bytes(dbl, cp, t));
@@ -362,7 +398,8 @@ BatchLayout batch_layout(const Batch& B, int64_t n) {
   BatchLayout l;
   l.pairs = 0;
   l.items = al(sizeof(BatchPair) * (size_t)std::max<int64_t>(n, 1));
-  l.counter = l.items + al(sizeof(int2) * std::max<size_t>(B.hitems.size(), 1));
+  l.bits = l.items + al(sizeof(int2) * std::max<size_t>(B.hitems.size(), 1));
+  l.counter = l.bits + al(sizeof(BitDesc) * B.hbits.size());
   l.tab = l.counter + 256;
   l.copy = l.tab + al(std::max<size_t>(B.htab.size(), 1) * sizeof(int64_t));
   l.tilecnt = l.copy;
@@ -378,6 +415,7 @@ void place_batch(Batch& B, const std::vector<const PlannedPair*>& lw, char* base
   const BatchLayout l = batch_layout(B, n);
   B.dpairs = (BatchPair*)(base + l.pairs);
   B.ditems = (int2*)(base + l.items);
+  B.dbits = (BitDesc*)(base + l.bits);
   B.dcounter = (int32_t*)(base + l.counter);
   B.dtilecnt = (int32_t*)(base + l.tilecnt);
   const int64_t* dtab = (const int64_t*)(base + l.tab);
@@ -387,6 +425,12 @@ void place_batch(Batch& B, const std::vector<const PlannedPair*>& lw, char* base
     BatchPair& P = B.hpairs[(size_t)i];
     std::memset(&P, 0, sizeof P);
     if (L.solo) continue;  // no tables, never in the work list
+    if (!B.bit_index.empty() && B.bit_index[(size_t)i] >= 0) {
+      BitDesc& q = B.hbits[(size_t)B.bit_index[(size_t)i]];
+      q.L = q.long_b ? L.b : L.a;
+      q.S = q.long_b ? L.a : L.b;
+      q.C = L.c;
+    }
     P.A = L.a;
     P.B = L.b;
     P.C = L.c;
@@ -413,15 +457,17 @@ void place_batch(Batch& B, const std::vector<const PlannedPair*>& lw, char* base
     for (int t = 0; t < 9; ++t) *tabs[t] = make_tab(tb, L.t[map[t]]);
   }
   const size_t np = sizeof(BatchPair) * (size_t)n, ni = sizeof(int2) * B.hitems.size(),
-               nt = B.htab.size() * sizeof(int64_t);
+               nt = B.htab.size() * sizeof(int64_t), nb = sizeof(BitDesc) * B.hbits.size();
   if (staging) {
     std::memcpy(staging + l.pairs, B.hpairs.data(), np);
     if (ni) std::memcpy(staging + l.items, B.hitems.data(), ni);
+    if (nb) std::memcpy(staging + l.bits, B.hbits.data(), nb);
     if (nt) std::memcpy(staging + l.tab, B.htab.data(), nt);
     MH_HIP_CHECK(hipMemcpyAsync(base, staging, l.copy, hipMemcpyHostToDevice, s));
   } else {
     if (np) MH_HIP_CHECK(hipMemcpy(base + l.pairs, B.hpairs.data(), np, hipMemcpyHostToDevice));
     if (ni) MH_HIP_CHECK(hipMemcpy(base + l.items, B.hitems.data(), ni, hipMemcpyHostToDevice));
+    if (nb) MH_HIP_CHECK(hipMemcpy(base + l.bits, B.hbits.data(), nb, hipMemcpyHostToDevice));
     if (nt) MH_HIP_CHECK(hipMemcpy(base + l.tab, B.htab.data(), nt, hipMemcpyHostToDevice));
   }
 }
@@ -464,7 +510,7 @@ std::unique_ptr<Batch> build_batch(Handle& h, int64_t n, const muscle_hip_tensor
 }
 
 void batch_launch(Batch& b, hipStream_t s) {
-  const int64_t nmain = (int64_t)b.hitems.size() - b.nsplit - b.nshallow - b.nskinny;
+  const int64_t nmain = (int64_t)b.hitems.size() - b.nsplit - b.nshallow - b.nskinny - b.nbits;
   if (nmain > 0 || b.nsplit > 0) {
     BatchArgs a;
     a.pairs = b.dpairs;
@@ -503,6 +549,13 @@ void batch_launch(Batch& b, hipStream_t s) {
     a.items = b.ditems + nmain + b.nsplit + b.nshallow;
     a.nitems = b.nskinny;
     launch_skinny(is_double(b.dtype), is_complex(b.dtype), a, s);
+  }
+  if (b.nbits > 0) {
+    BitArgs a;
+    a.descs = b.dbits;
+    a.items = b.ditems + nmain + b.nsplit + b.nshallow + b.nskinny;
+    a.nitems = b.nbits;
+    launch_bits(is_double(b.dtype), is_complex(b.dtype), a, b.bits_lds, s);
   }
 }
 
@@ -582,7 +635,8 @@ void batch_autotune(Batch& b, int samples, int reps) {
   for (size_t i = 0; i < b.hpairs.size(); ++i) {
     const BatchPair& P = b.hpairs[i];
     if (P.M * (int64_t)P.N * P.NB == 0 || (i < b.solo.size() && b.solo[i])) continue;
-    if (b.pinfo[i].route == MUSCLE_HIP_PAIR_SKINNY) continue;  // no tile shape to choose
+    // no tile shape to choose
+    if (b.pinfo[i].route == MUSCLE_HIP_PAIR_SKINNY || b.bit_index[i] >= 0) continue;
     by_class[tuning_class(P.M, P.N)].push_back((int64_t)i);
   }
   hipEvent_t e0, e1;
@@ -677,16 +731,16 @@ int muscle_hip_batch_get_info(muscle_hip_batch_t batch, muscle_hip_batch_info_t*
     Batch* b = reinterpret_cast<Batch*>(batch);
     if (!b || !info) fail(MUSCLE_HIP_INVALID_ARGUMENT, "null batch or info");
     info->pairs = (int64_t)b->cs.size();
-    info->items = (int64_t)b->hitems.size();
-    info->shallow_items = b->nshallow;
-    info->skinny_items = b->nskinny;
+    info->items = b->all_tiles;
+    info->shallow_items = b->shallow_tiles;
+    info->skinny_items = b->skinny_tiles;
     info->split_items = b->split_items;
     info->workgroups = b->workgroups;
     info->graph = b->exec ? 1 : 0;
     info->flops = b->flops;
     info->bytes = b->bytes;
     info->table_bytes = (int64_t)(b->htab.size() * 8 + b->hpairs.size() * sizeof(BatchPair) +
-                                  b->hitems.size() * sizeof(int2));
+                                  b->hitems.size() * sizeof(int2) + b->hbits.size() * sizeof(BitDesc));
   });
 }
 

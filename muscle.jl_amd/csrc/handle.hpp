@@ -10,6 +10,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "bits.hpp"
 #include "kernels.hpp"
 #include "lowering.hpp"
 
@@ -20,7 +21,7 @@ enum TabId { TAB_ROWA = 0, TAB_KA, TAB_KB, TAB_COLB, TAB_ROWC, TAB_COLC, TAB_BA,
 
 // A lowered contraction with its offset tables resident on the device.
 struct Plan {
-  enum Kind { EMPTY = 0, GEMM = 1, REDUCE = 2, SPLIT = 3, PERMUTE = 4 };
+  enum Kind { EMPTY = 0, GEMM = 1, REDUCE = 2, SPLIT = 3, PERMUTE = 4, BITS = 5 };
   int kind = EMPTY;
   int precision = MUSCLE_HIP_PRECISION_NATIVE;
   ContractionDesc d;
@@ -54,6 +55,8 @@ struct Plan {
   bool pack_a = false, pack_b = false;
   bool pack_a_kfast = false, pack_b_kfast = false;  // read order of the pack tiles
   std::unique_ptr<Plan> inner;
+  // power-of-two kernel: everything but the addresses
+  BitDesc bits;
   // reduction kernel configuration
   int gshift = 0;
   int nsplit = 1;

@@ -266,6 +266,173 @@ void check_ktiles(std::mt19937_64& rng) {
   std::printf("%lld tile GEMM plans checked, %lld K-tile sizes with a common base\n", (long long)plans, (long long)set);
 }
 
+// The power-of-two kernel's plan, run on the host index by index as the kernel
+// does: every element lies inside its operand, the LDS copies are one-to-one,
+// and C equals the naive sum over all labels, each output written once.
+void check_bits(std::mt19937_64& rng) {
+  int planned = 0, chunked = 0;
+  for (int it = 0; it < 120; ++it) {
+    std::vector<int64_t> extent(1, 1);
+    std::vector<int32_t> la, lb, lc;
+    auto label = [&](int64_t e) {
+      extent.push_back(e);
+      return (int32_t)extent.size() - 1;
+    };
+    // 11 to 14 output bits, mostly in modes of two, split unevenly over the
+    // classes; 0 to 7 contracted bits
+    int bits = 11 + (int)(rng() % 4), kbits = (int)(rng() % 8);
+    const int pn = (int)(rng() % 11), nh = (int)(rng() % 3);
+    for (int h = 0; h < nh; ++h) {
+      const int32_t l = label(2);
+      la.push_back(l);
+      lb.push_back(l);
+      lc.push_back(l);
+    }
+    bits -= nh;
+    while (bits > 0) {
+      const int w = std::min<int>(bits, rng() % 4 == 0 ? 3 : 1);
+      const int32_t l = label(int64_t(1) << w);
+      ((int)(rng() % 10) < pn ? lb : la).push_back(l);
+      lc.push_back(l);
+      bits -= w;
+    }
+    while (kbits > 0) {
+      const int w = std::min<int>(kbits, rng() % 4 == 0 ? 2 : 1);
+      const int32_t l = label(int64_t(1) << w);
+      la.push_back(l);
+      lb.push_back(l);
+      kbits -= w;
+    }
+    Operand a = make_operand(la, extent, rng), b = make_operand(lb, extent, rng), c = make_operand(lc, extent, rng);
+    const int dt = (int)(rng() % 4);
+    const muscle_hip_tensor_t tc = c.desc(dt, (void*)256), ta = a.desc(dt, (void*)256), tb = b.desc(dt, (void*)256);
+    const mh::ContractionDesc d = mh::lower_binary(tc, ta, tb);
+    mh::BitDesc q;
+    if (!mh::plan_bits(d, q)) continue;
+    ++planned;
+    chunked += q.nchunk > 1;
+    q.run = std::min(q.tiles, 4);  // large launches run several tiles per workgroup
+    // kernel operands (after the lowering's exchange)
+    const Operand &A = d.swapped ? b : a, &B = d.swapped ? a : b;
+    const Operand &L = q.long_b ? B : A, &S = q.long_b ? A : B;
+    std::vector<int64_t> vl((size_t)L.span), vs((size_t)S.span), vc((size_t)c.span, 0), ref((size_t)c.span, 0);
+    std::vector<char> seen((size_t)c.span, 0);
+    for (auto& x : vl) x = (int64_t)(rng() % 201) - 100;
+    for (auto& x : vs) x = (int64_t)(rng() % 201) - 100;
+    const int FL = 1 << q.reg_long, FS = 1 << (mh::kBitReg - q.reg_long);
+    auto bit_sum = [](uint32_t t, const uint32_t* s, int n) {
+      uint32_t o = 0;
+      for (int j = 0; j < n; ++j)
+        if (t >> j & 1) o += s[j];
+      return o;
+    };
+    auto bit_xor = [](uint32_t t, const uint32_t* s, int n) {
+      uint32_t o = 0;
+      for (int j = 0; j < n; ++j)
+        if (t >> j & 1) o ^= s[j];
+      return o;
+    };
+    bool inside = true, once = true, steps = true;
+    const int NT = 1 << mh::kBitThread;
+    for (uint32_t t0 = 0; t0 < (uint32_t)q.tiles; t0 += (uint32_t)q.run) {
+      uint32_t oL = bit_sum(t0, q.oL, 32), oS = bit_sum(t0, q.oS, 32), oC = bit_sum(t0, q.oC, 32);
+      for (uint32_t t = t0; t < t0 + (uint32_t)q.run; ++t) {
+        std::vector<int64_t> acc((size_t)NT * 8, 0);
+        uint32_t kL = 0, kS = 0;
+        for (int ch = 0; ch < q.nchunk; ++ch) {
+          std::vector<int64_t> ll((size_t)q.nl, 0), ls((size_t)q.ns, 0);
+          std::vector<char> wl((size_t)q.nl, 0), ws((size_t)q.ns, 0);
+          for (int tid = 0; tid < NT; ++tid) {
+            for (int i = 0; i < mh::kBitLongIt; ++i) {
+              if (!(i == 0 ? tid < q.nl : i * NT < q.nl)) continue;
+              const uint64_t o = (uint64_t)(uint32_t)(oL + kL) + q.iL[i] + bit_sum((uint32_t)tid, q.gL, 8);
+              const uint32_t x = bit_xor((uint32_t)tid, q.gLl, 8) ^ q.iLl[i];
+              if (o >= vl.size() || x >= ll.size()) {
+                inside = false;
+                continue;
+              }
+              once = once && !wl[x];
+              wl[x] = 1;
+              ll[x] = vl[o];
+            }
+            for (int i = 0; i < mh::kBitShortIt; ++i) {
+              if (!(i == 0 ? tid < q.ns : i * NT < q.ns)) continue;
+              const uint64_t o = (uint64_t)(uint32_t)(oS + kS) + q.iS[i] + bit_sum((uint32_t)tid, q.gS, 8);
+              const uint32_t x = bit_xor((uint32_t)tid, q.gSl, 8) ^ q.iSl[i];
+              if (o >= vs.size() || x >= ls.size()) {
+                inside = false;
+                continue;
+              }
+              once = once && !ws[x];
+              ws[x] = 1;
+              ls[x] = vs[o];
+            }
+          }
+          if (ch + 1 < q.nchunk) {
+            kL += q.cL[__builtin_ctz(ch + 1)];
+            kS += q.cS[__builtin_ctz(ch + 1)];
+          }
+          for (int tid = 0; tid < NT; ++tid)
+            for (int i = 0; i < FL; ++i)
+              for (int j = 0; j < FS; ++j)
+                for (int k = 0; k < q.kc; ++k) {
+                  const uint32_t x = ((bit_xor((uint32_t)tid, q.tL, 8) ^ bit_xor((uint32_t)i, q.rX, q.reg_long)) ^
+                                      ((uint32_t)k & (uint32_t)q.kxl)) + (uint32_t)(k * q.sl);
+                  const uint32_t y = ((bit_xor((uint32_t)tid, q.tS, 8) ^
+                                       bit_xor((uint32_t)j, q.rX + q.reg_long, mh::kBitReg - q.reg_long)) ^
+                                      ((uint32_t)k & (uint32_t)q.kxs)) + (uint32_t)(k * q.ss);
+                  if (x >= ll.size() || y >= ls.size()) {
+                    inside = false;
+                    continue;
+                  }
+                  acc[(size_t)tid * 8 + (size_t)(i * FS + j)] += ll[x] * ls[y];
+                }
+        }
+        for (int tid = 0; tid < NT; ++tid)
+          for (int i = 0; i < FL; ++i)
+            for (int j = 0; j < FS; ++j) {
+              const uint64_t o = (uint64_t)oC + bit_sum((uint32_t)tid, q.tC, 8) + bit_sum((uint32_t)i, q.rC, q.reg_long) +
+                                 bit_sum((uint32_t)j, q.rC + q.reg_long, mh::kBitReg - q.reg_long);
+              if (o >= vc.size()) {
+                inside = false;
+                continue;
+              }
+              once = once && !seen[o];
+              seen[o] = 1;
+              vc[o] = acc[(size_t)tid * 8 + (size_t)(i * FS + j)];
+            }
+        if (t + 1 < t0 + (uint32_t)q.run) {
+          const int j = __builtin_ctz(t + 1);
+          oL += q.sL[j];
+          oS += q.sS[j];
+          oC += q.sC[j];
+          steps = steps && oL == bit_sum(t + 1, q.oL, 32) && oS == bit_sum(t + 1, q.oS, 32) &&
+                  oC == bit_sum(t + 1, q.oC, 32);
+        }
+      }
+    }
+    expect(inside, "power-of-two plan: an index outside its buffer", it);
+    expect(once, "power-of-two plan: an element written twice", it);
+    expect(steps, "power-of-two plan: tile steps", it);
+    // naive sum over all label assignments
+    std::vector<int64_t> idx(extent.size(), 0);
+    auto off = [&](const Operand& o) {
+      int64_t r = 0;
+      for (size_t i = 0; i < o.modes.size(); ++i) r += idx[(size_t)o.modes[i]] * o.strides[i];
+      return (size_t)r;
+    };
+    for (;;) {
+      ref[off(c)] += vl[off(L)] * vs[off(S)];
+      size_t l = 1;
+      while (l < extent.size() && ++idx[l] == extent[l]) idx[l++] = 0;
+      if (l == extent.size()) break;
+    }
+    expect(vc == ref, "power-of-two plan: result", it);
+  }
+  expect(planned > 80 && chunked > 10, "power-of-two plans", planned);
+  std::printf("power-of-two kernel: %d plans run on the host, %d with K chunks\n", planned, chunked);
+}
+
 bool is_cplx(int dt) { return dt == MUSCLE_HIP_C32 || dt == MUSCLE_HIP_C64; }
 
 std::vector<char> encode(const std::vector<cd>& v, int dt) {
@@ -518,6 +685,7 @@ int main(int argc, char** argv) {
   check_describe(rng);
   std::mt19937_64 rng_k(20261204);
   check_ktiles(rng_k);
+  check_bits(rng_k);
   if (argc > 1 && std::strcmp(argv[1], "--gpu") == 0) check_gpu(rng);
   std::printf("%s: %d failures\n", g_failures ? "FAILED" : "ok", g_failures);
   return g_failures ? 1 : 0;
