@@ -10,8 +10,10 @@
 // contraction of every admitted job whose operands have been launched
 // (stream order makes them complete first): contractions big enough to fill
 // the GPU alone take the single-contraction kernel, all others share one
-// persistent batched launch per element type.  Up to kSlots ticks are in
-// flight; when a tick's event fires, operands that have no consumer left go
+// persistent batched launch per element type, the double-precision types on
+// one stream and the single-precision ones on another (a job has one element
+// type, so the two never read each other's results).  Up to kSlots ticks are in
+// flight; when a tick's events fire, operands that have no consumer left go
 // back to the pool and the owning job's reservation shrinks, so waiting jobs
 // are admitted while others are still on the GPU.  Mode 1 runs the same jobs
 // as the plain per-call loop (one job at a time, one launch per node).
@@ -92,15 +94,39 @@ class Pool {
   std::map<size_t, size_t> free_;
 };
 
+// Memory of a job's mode, extent and stride lists: blocks given back together.
+class Arena {
+ public:
+  template <typename T>
+  T* alloc(size_t n) {
+    const size_t bytes = (n * sizeof(T) + 7) & ~size_t(7);
+    if (bytes > left_) {
+      left_ = std::max(bytes, kBlock);
+      blocks_.emplace_back(new char[left_]);
+      at_ = blocks_.back().get();
+    }
+    T* p = reinterpret_cast<T*>(at_);
+    at_ += bytes;
+    left_ -= bytes;
+    return p;
+  }
+
+ private:
+  static constexpr size_t kBlock = size_t(64) << 10;
+  std::vector<std::unique_ptr<char[]>> blocks_;
+  char* at_ = nullptr;
+  size_t left_ = 0;
+};
+
 struct Operand {
-  muscle_hip_tensor_t t;
-  std::vector<int32_t> modes;
-  std::vector<int64_t> ext, str;
-  void fix() {
-    t.modes = modes.data();
-    t.extents = ext.data();
-    t.strides = str.data();
-    t.rank = (int32_t)modes.size();
+  muscle_hip_tensor_t t{};  // its lists are in the job's arena
+  int32_t* modes = nullptr;
+  int64_t *ext = nullptr, *str = nullptr;
+  void init(Arena& a, int rank) {
+    t.rank = (int32_t)rank;
+    t.modes = modes = a.alloc<int32_t>((size_t)rank);
+    t.extents = ext = a.alloc<int64_t>((size_t)rank);
+    t.strides = str = a.alloc<int64_t>((size_t)rank);
   }
 };
 
@@ -112,7 +138,6 @@ struct Node {
   std::vector<int> users;  // nodes that read this node's output
   int pending = 0;         // node operands not launched yet
   bool solo = false;       // runs as a single-contraction launch
-  PlannedPair plan;        // batched nodes: lowering, tables, tile
   bool launched = false, done = false, freed = false;
 };
 
@@ -121,6 +146,7 @@ enum CompileState { kQueued = 0, kCompiled = 1, kFailed = 2 };
 struct Job {
   int64_t id = 0;
   int dtype = 0;
+  Arena lists;
   std::vector<Operand> leaves;
   std::vector<Node> nodes;
   size_t reserve = 0;   // bytes of all intermediates, the result and the tables
@@ -135,6 +161,8 @@ struct Job {
   double t_submit = 0, t_admit = 0, t_done = 0;
   int64_t ticks = 0;
   int remaining = 0;
+  std::vector<PlannedPair> plans;  // per node: lowering and, batched, tables and tile; until all are launched
+  int unlaunched = 0;
   const Operand& operand(int k) const {
     const int nl = (int)leaves.size();
     return k < nl ? leaves[(size_t)k] : nodes[(size_t)(k - nl)].out;
@@ -150,7 +178,8 @@ struct Slot {
   char* dev = nullptr;
   char* pinned = nullptr;
   size_t size = 0;
-  hipEvent_t ev = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};  // per lane
+  bool used[2] = {false, false};
   std::vector<TickEntry> entries;
   std::vector<std::unique_ptr<Batch>> batches;
   std::vector<void*> extra_dev;  // oversized tick descriptors
@@ -166,12 +195,20 @@ constexpr int kMaxPlanners = 8;
 
 struct Server {
   Handle h;
+  // the single-precision jobs' stream, plans and workspace: a tick's launches
+  // are short chains of few workgroups, so two element types one after the
+  // other leave most of the GPU idle (24 jobs of both, 20 to 300 contractions
+  // each: 8 ms of launches in a row of 10 ms, side by side 5)
+  Handle hs;
   int mode = 0;
   int max_active = 64;
   std::mutex mu;
   std::condition_variable cv_work, cv_done, cv_plan;
   std::deque<std::shared_ptr<Job>> waiting;   // arrival order, compiled or not
   std::deque<std::shared_ptr<Job>> to_compile;
+  // every contraction launched: the planner threads free the plans while the
+  // GPU works (24 jobs' plans held up the releases for 2 of 3 ms)
+  std::vector<std::shared_ptr<Job>> launched;
   std::vector<std::shared_ptr<Job>> active;
   std::unordered_map<int64_t, std::shared_ptr<Job>> jobs;
   Pool pool;
@@ -185,6 +222,9 @@ struct Server {
   muscle_hip_server_stats_t st{};
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
   std::string worker_error;
+
+  static int lane_of(int dtype) { return is_double(dtype) ? 0 : 1; }
+  Handle& lane(int i) { return i == 0 ? h : hs; }
 
   double now() const {
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -204,9 +244,8 @@ struct Server {
 namespace {
 
 void column_major(Operand& o) {
-  o.str.resize(o.ext.size());
   int64_t s = 1;
-  for (size_t i = 0; i < o.ext.size(); ++i) {
+  for (int i = 0; i < o.t.rank; ++i) {
     o.str[i] = s;
     s *= std::max<int64_t>(o.ext[i], 1);
   }
@@ -214,7 +253,7 @@ void column_major(Operand& o) {
 
 int64_t elems(const Operand& o) {
   int64_t n = 1;
-  for (int64_t e : o.ext) n *= e;
+  for (int i = 0; i < o.t.rank; ++i) n *= o.ext[i];
   return n;
 }
 
@@ -222,13 +261,16 @@ int64_t elems(const Operand& o) {
 
 // Lowers every contraction of a job; the batched ones get tables and a tile.
 void Server::compile(Job& j) {
-  for (Node& nd : j.nodes) {
+  j.plans.resize(j.nodes.size());
+  for (size_t i = 0; i < j.nodes.size(); ++i) {
+    Node& nd = j.nodes[i];
+    PlannedPair& plan = j.plans[i];
     muscle_hip_tensor_t c = nd.out.t;
     c.data = (void*)256;  // addresses are bound at launch; the lowering reads shapes and strides only
-    nd.plan.d = lower_binary(c, j.operand(nd.lhs).t, j.operand(nd.rhs).t);
-    const ContractionDesc& d = nd.plan.d;
+    plan.d = lower_binary(c, j.operand(nd.lhs).t, j.operand(nd.rhs).t);
+    const ContractionDesc& d = plan.d;
     nd.solo = (double)d.M * (double)d.N * (double)d.K * (double)d.B >= kSoloPoints;
-    if (!nd.solo) plan_pair(h, nd.plan, j.htab, MUSCLE_HIP_TILE_AUTO, kTickSingleMax);
+    if (!nd.solo) plan_pair(h, plan, j.htab, MUSCLE_HIP_TILE_AUTO, kTickSingleMax);
   }
   j.dtab_bytes = j.htab.empty() ? 0 : al256(j.htab.size() * sizeof(int64_t));
 }
@@ -238,7 +280,14 @@ void Server::plan_loop() {
     std::shared_ptr<Job> j;
     {
       std::unique_lock<std::mutex> lk(mu);
-      cv_plan.wait(lk, [&] { return stop || !to_compile.empty(); });
+      cv_plan.wait(lk, [&] { return stop || !to_compile.empty() || !launched.empty(); });
+      if (!launched.empty()) {
+        j = launched.back();
+        launched.pop_back();
+        lk.unlock();
+        std::vector<PlannedPair>().swap(j->plans);
+        continue;
+      }
       if (to_compile.empty()) return;  // stopping
       j = to_compile.front();
       to_compile.pop_front();
@@ -374,9 +423,11 @@ bool Server::launch_tick() {
     }
   }
   if (entries.empty()) return false;
+  int drops = 0;
   Slot& sl = slots[(slot_head + slot_count) % kSlots];
   sl.entries = entries;
   sl.batches.clear();
+  sl.used[0] = sl.used[1] = false;
   size_t used = 0;
   std::vector<const PlannedPair*> lw[MUSCLE_HIP_C64 + 1];
   for (const TickEntry& e : entries) {
@@ -385,12 +436,14 @@ bool Server::launch_tick() {
     const muscle_hip_tensor_t& a = j.operand(nd.lhs).t;
     const muscle_hip_tensor_t& b = j.operand(nd.rhs).t;
     if (nd.solo) {
-      Plan* pl = get_plan(h, 1, MUSCLE_HIP_PRECISION_NATIVE, 1e-12, &nd.out.t, &a, &b);
-      run_contraction(h, *pl, nd.out.t, a, &b);
+      Handle& lh = lane(lane_of(j.dtype));
+      Plan* pl = get_plan(lh, 1, MUSCLE_HIP_PRECISION_NATIVE, 1e-12, &nd.out.t, &a, &b);
+      run_contraction(lh, *pl, nd.out.t, a, &b);
+      sl.used[lane_of(j.dtype)] = true;
       st.launched_pairs++;
       continue;
     }
-    PlannedPair& L = nd.plan;
+    PlannedPair& L = j.plans[(size_t)e.node];
     L.a = L.d.swapped ? b.data : a.data;
     L.b = L.d.swapped ? a.data : b.data;
     L.c = nd.out.t.data;
@@ -399,27 +452,41 @@ bool Server::launch_tick() {
   }
   for (int dt = MUSCLE_HIP_F32; dt <= MUSCLE_HIP_C64; ++dt) {
     if (lw[dt].empty()) continue;
+    const hipStream_t stream = lane(lane_of(dt)).stream;
+    sl.used[lane_of(dt)] = true;
     std::unique_ptr<Batch> B(new Batch());
     B->h = &h;
     B->dtype = dt;
     finish_batch(h, *B, lw[dt]);
     const BatchLayout l = batch_layout(*B, (int64_t)lw[dt].size());
     if (used + l.total <= sl.size) {
-      place_batch(*B, lw[dt], sl.dev + used, sl.pinned + used, h.stream);
+      place_batch(*B, lw[dt], sl.dev + used, sl.pinned + used, stream);
       used += al256(l.total);
     } else {
       void* d = nullptr;
       if (hipMalloc(&d, l.total) != hipSuccess) fail(MUSCLE_HIP_OUT_OF_MEMORY, "tick descriptors");
       sl.extra_dev.push_back(d);
-      place_batch(*B, lw[dt], (char*)d, nullptr, h.stream);
+      place_batch(*B, lw[dt], (char*)d, nullptr, stream);
     }
-    if (!B->hitems.empty()) batch_launch(*B, h.stream);
+    if (!B->hitems.empty()) batch_launch(*B, stream);
     MH_HIP_CHECK(hipGetLastError());
     B->h = nullptr;  // completion is tracked by the slot event
     st.launched_pairs += (int64_t)lw[dt].size();
     sl.batches.push_back(std::move(B));
   }
-  MH_HIP_CHECK(hipEventRecord(sl.ev, h.stream));
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    for (auto& e : entries) e.job->unlaunched--;
+    for (auto& jp : active)
+      if (jp->unlaunched == 0) {
+        jp->unlaunched = -1;
+        launched.push_back(jp);
+        ++drops;
+      }
+  }
+  if (drops) cv_plan.notify_all();
+  for (int i = 0; i < 2; ++i)
+    if (sl.used[i]) MH_HIP_CHECK(hipEventRecord(sl.ev[i], lane(i).stream));
   slot_count++;
   st.ticks++;
   return true;
@@ -430,7 +497,9 @@ bool Server::complete_ticks(bool block) {
   bool any = false;
   while (slot_count > 0) {
     Slot& sl = slots[slot_head];
-    hipError_t q = block && !any ? hipEventSynchronize(sl.ev) : hipEventQuery(sl.ev);
+    hipError_t q = hipSuccess;
+    for (int i = 0; i < 2 && q == hipSuccess; ++i)
+      if (sl.used[i]) q = block && !any ? hipEventSynchronize(sl.ev[i]) : hipEventQuery(sl.ev[i]);
     if (q == hipErrorNotReady) break;
     if (q != hipSuccess) fail(MUSCLE_HIP_HIP_ERROR, std::string("tick: ") + hipGetErrorString(q));
     {
@@ -508,7 +577,7 @@ void Server::loop() {
       for (auto& j : admitted)
         if (j->dtab_bytes)
           MH_HIP_CHECK(hipMemcpyAsync(j->dtab, j->htab.data(), j->htab.size() * sizeof(int64_t),
-                                      hipMemcpyHostToDevice, h.stream));
+                                      hipMemcpyHostToDevice, lane(lane_of(j->dtype)).stream));
       if (mode == 1) {
         std::shared_ptr<Job> j;
         {
@@ -569,12 +638,13 @@ int guarded_s(F&& f) {
   }
 }
 
-void copy_operand(Operand& o, const muscle_hip_tensor_t& t) {
-  o.t = t;
-  o.modes.assign(t.modes, t.modes + t.rank);
-  o.ext.assign(t.extents, t.extents + t.rank);
-  o.str.assign(t.strides, t.strides + t.rank);
-  o.fix();
+void copy_operand(Arena& lists, Operand& o, const muscle_hip_tensor_t& t) {
+  o.init(lists, t.rank);
+  o.t.dtype = t.dtype;
+  o.t.data = t.data;
+  std::copy(t.modes, t.modes + t.rank, o.modes);
+  std::copy(t.extents, t.extents + t.rank, o.ext);
+  std::copy(t.strides, t.strides + t.rank, o.str);
 }
 }  // namespace
 
@@ -586,7 +656,8 @@ int muscle_hip_server_create(int64_t pool_bytes, int max_active_jobs, int mode, 
     if (pool_bytes <= 0 || mode < 0 || mode > 1) fail(MUSCLE_HIP_INVALID_ARGUMENT, "bad pool size or mode");
     std::unique_ptr<Server> S(new Server());
     MH_HIP_CHECK(hipGetDevice(&S->h.device));
-    MH_HIP_CHECK(hipStreamCreateWithFlags(&S->h.stream, hipStreamNonBlocking));
+    S->hs.device = S->h.device;
+    for (int i = 0; i < 2; ++i) MH_HIP_CHECK(hipStreamCreateWithFlags(&S->lane(i).stream, hipStreamNonBlocking));
     S->mode = mode;
     S->max_active = std::max(1, max_active_jobs);
     if (hipMalloc(&S->arena, (size_t)pool_bytes) != hipSuccess) {
@@ -598,7 +669,7 @@ int muscle_hip_server_create(int64_t pool_bytes, int max_active_jobs, int mode, 
     for (Slot& sl : S->slots) {
       MH_HIP_CHECK(hipMalloc(&sl.dev, kSlotBytes));
       MH_HIP_CHECK(hipHostMalloc((void**)&sl.pinned, kSlotBytes, hipHostMallocDefault));
-      MH_HIP_CHECK(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming));
+      for (hipEvent_t& ev : sl.ev) MH_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
       sl.size = kSlotBytes;
     }
     S->st.pool_bytes = pool_bytes;
@@ -621,7 +692,7 @@ int muscle_hip_server_submit(muscle_hip_server_t server, const muscle_hip_job_t*
     j->leaves.resize((size_t)job->n_leaves);
     for (int i = 0; i < job->n_leaves; ++i) {
       check_tensor(&job->leaves[i], "leaf");
-      copy_operand(j->leaves[(size_t)i], job->leaves[i]);
+      copy_operand(j->lists, j->leaves[(size_t)i], job->leaves[i]);
     }
     j->dtype = job->leaves[0].dtype;
     for (int i = 1; i < job->n_leaves; ++i)
@@ -637,15 +708,14 @@ int muscle_hip_server_submit(muscle_hip_server_t server, const muscle_hip_job_t*
         fail(MUSCLE_HIP_INVALID_ARGUMENT, "node operands must precede the node");
       const int o0 = job->node_off[i], o1 = job->node_off[i + 1];
       if (o0 < 0 || o1 < o0) fail(MUSCLE_HIP_INVALID_ARGUMENT, "bad node_off");
-      nd.out.modes.assign(job->node_modes + o0, job->node_modes + o1);
-      for (int32_t m : nd.out.modes) {
+      nd.out.init(j->lists, o1 - o0);
+      for (int x = 0; x < o1 - o0; ++x) {
+        const int32_t m = nd.out.modes[x] = job->node_modes[o0 + x];
         if (m < 0 || m >= job->n_labels) fail(MUSCLE_HIP_INVALID_ARGUMENT, "mode label out of range");
-        nd.out.ext.push_back(job->label_extents[m]);
+        nd.out.ext[x] = job->label_extents[m];
       }
       column_major(nd.out);
       nd.out.t.dtype = j->dtype;
-      nd.out.t.data = nullptr;
-      nd.out.fix();
       nd.bytes = (size_t)elems(nd.out) * es;
       j->reserve += al256(std::max<size_t>(nd.bytes, 1));
       (void)total;
@@ -664,7 +734,7 @@ int muscle_hip_server_submit(muscle_hip_server_t server, const muscle_hip_job_t*
     }
     // the root is consumed by the caller (muscle_hip_server_release)
     j->nodes.back().consumers++;
-    j->remaining = job->n_nodes;
+    j->remaining = j->unlaunched = job->n_nodes;
     {
       std::lock_guard<std::mutex> lk(S->mu);
       S->st.submitted++;
@@ -738,10 +808,12 @@ int muscle_hip_server_release(muscle_hip_server_t server, int64_t job_id) {
   return guarded_s([&] {
     Server* S = reinterpret_cast<Server*>(server);
     if (!S) fail(MUSCLE_HIP_INVALID_ARGUMENT, "null server");
+    std::shared_ptr<Job> keep;  // freed after the lock
     std::lock_guard<std::mutex> lk(S->mu);
     auto it = S->jobs.find(job_id);
     if (it == S->jobs.end()) fail(MUSCLE_HIP_INVALID_ARGUMENT, "unknown job");
-    Job& j = *it->second;
+    keep = it->second;
+    Job& j = *keep;
     if (j.status == MUSCLE_HIP_NOT_READY) fail(MUSCLE_HIP_NOT_READY, "job still running");
     Node& root = j.nodes.back();
     if (j.status == MUSCLE_HIP_OK && !root.freed && root.out.t.data) {
@@ -785,16 +857,20 @@ int muscle_hip_server_destroy(muscle_hip_server_t server) {
     S->cv_plan.notify_all();
     for (auto& t : S->planners) t.join();
     if (S->worker.joinable()) S->worker.join();
-    (void)hipStreamSynchronize(S->h.stream);
+    for (int i = 0; i < 2; ++i) (void)hipStreamSynchronize(S->lane(i).stream);
     for (Slot& sl : S->slots) {
       if (sl.dev) (void)hipFree(sl.dev);
       if (sl.pinned) (void)hipHostFree(sl.pinned);
-      if (sl.ev) (void)hipEventDestroy(sl.ev);
+      for (hipEvent_t ev : sl.ev)
+        if (ev) (void)hipEventDestroy(ev);
     }
     if (S->arena) (void)hipFree(S->arena);
-    S->h.cache.clear();
-    (void)hipStreamDestroy(S->h.stream);
-    S->h.stream = nullptr;
+    for (int i = 0; i < 2; ++i) {
+      Handle& lh = S->lane(i);
+      lh.cache.clear();
+      (void)hipStreamDestroy(lh.stream);
+      lh.stream = nullptr;
+    }
     delete S;
   });
 }
