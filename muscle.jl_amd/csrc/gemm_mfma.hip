@@ -543,6 +543,10 @@ void launch_tile(GemmArgs g, hipStream_t s) {
 //     workgroups per CU in place of three, half the barriers);
 //   real FP64, 64x64x16 / 32x32x16: 1024: 32 / 26, 1536: 58 / 52, 2048: 75 / 88;
 //   ComplexF32, 64x64x8 / 32x64x16: 1024: 46 / 34, 1536: 75 / 76, 2048: 101 / 110;
+//     where K's modes leave no common base per K-tile (a lookup per k, fewer of
+//     them in a longer K-tile), 64x64x16 / 32x64x16: 1728 x 1728 x 1728 (729 tiles)
+//     339 / 377, and against 64x64x8 2197 x 2197 x 2197 710 / 801, but with K
+//     sliced (1000 x 1000 x 2197) 187 / 162;
 //   real FP32, 64x64x16 / 32x64x16: 1024: 22 / 17, 1536: 35 / 30, 2048: 43 / 49.
 template <typename T, typename S, bool CA, bool CB, bool G3>
 void launch_t(const GemmArgs& g, hipStream_t s) {
@@ -562,7 +566,9 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
       else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 4, 1>>(g, s);
     }
   } else if constexpr (CA || CB) {
-    if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
+    const bool lookups = !g.ktile8 && g.ksplit == 1;
+    if (tiles < (lookups ? 640 : 1024)) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
+    else if (lookups) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 3, 1>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, sizeof(S) == 8 ? 3 : 4, 1>>(g, s);
   } else {
     if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
