@@ -95,7 +95,9 @@ void copy_desc(Batch& b, const muscle_hip_tensor_t& t, std::vector<muscle_hip_te
 // most is fetching its code and descriptors once, the others for 12 and 20.
 // A longer K is a chain of gathers: 2^3 x 2^8 x 2^7 (x 4) on its 4 tiles took
 // 60 us longer than the skinny kernel when its operands were in HBM, so from
-// 512 tiles on, as for a single contraction.
+// 512 tiles on, as for a single contraction; and a small pair's K in at most 4
+// chunks (60 pairs to rank 20: 1232 us without this, 1161 with it, as by the
+// other kernels alone).
 bool bits_pair(const ContractionDesc& d, bool others) {
   const double tiles = (double)d.M * (double)d.N * (double)d.B / (1 << kBitTile);
   if (d.K <= kShallowK) return others || tiles >= kBitMinTiles;
@@ -270,7 +272,7 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
         for (int64_t t = 0; t < items; ++t) xq[x].push_back(make_int2((int)i, (int)t));
         xload[x] += cost * (double)items;
       }
-    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small)))) {
+    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small) && small.nchunk <= kBitSmallChunks))) {
       const int32_t x = (int32_t)B.hbits.size();
       B.bit_index[(size_t)i] = x;
       B.hbits.push_back(L.bits ? L.bit : small);
