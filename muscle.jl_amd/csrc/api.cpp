@@ -169,11 +169,12 @@ void offset_range(const std::vector<Dim>& v, int w, int64_t& lo, int64_t& hi) {
   for (auto& x : v) (x.s[w] < 0 ? lo : hi) += (x.extent - 1) * x.s[w];
 }
 
+}  // namespace
+
 // The tile GEMM's per-K-tile addressing (GemmArgs::ktile8): element spans of a
 // K-tile in A and B from the rows' (columns') range and the first 16 k.
-void plan_gemm_ktiles(Plan& p) {
-  const ContractionDesc& d = p.d;
-  if (p.kind != Plan::GEMM) return;
+KTiles k_tiles(const ContractionDesc& d) {
+  KTiles r;
   int64_t span[2];
   for (int w = 0; w < 2; ++w) {
     int64_t lo, hi, klo = 0, khi = 0;
@@ -187,13 +188,25 @@ void plan_gemm_ktiles(Plan& p) {
       n *= x.extent;
     }
     offset_range(head, w, klo, khi);
-    (w == 0 ? p.min_a : p.min_b) = lo + klo;
+    (w == 0 ? r.min_a : r.min_b) = lo + klo;
     span[w] = (hi + khi - lo - klo + 1) * (int64_t)dtype_size(make_dtype(is_double(d.dt[2]), is_complex(d.dt[w])));
   }
   const int64_t lim = int64_t(1) << 32;
   const bool fits = span[0] < lim && span[1] < lim;
-  p.ktile8 = fits && splits_at(d.k, 8);
-  p.ktile16 = fits && splits_at(d.k, 16);
+  r.ktile8 = fits && splits_at(d.k, 8);
+  r.ktile16 = fits && splits_at(d.k, 16);
+  return r;
+}
+
+namespace {
+
+void plan_gemm_ktiles(Plan& p) {
+  if (p.kind != Plan::GEMM) return;
+  const KTiles t = k_tiles(p.d);
+  p.ktile8 = t.ktile8;
+  p.ktile16 = t.ktile16;
+  p.min_a = t.min_a;
+  p.min_b = t.min_b;
 }
 
 // The contraction runs in its operands' own precision (no ladder rung).

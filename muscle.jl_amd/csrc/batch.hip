@@ -42,6 +42,16 @@ struct Mma<float> {
   static __device__ inline int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
+// A work item and its pair's descriptor, the same for the whole workgroup: read
+// through the scalar cache.
+__device__ __forceinline__ int2 uniform_item(const int2* p) {
+  const int2 w = *p;
+  return make_int2(__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y));
+}
+__device__ __forceinline__ const BatchPair& uniform_pair(const BatchPair* p) {
+  return *(const BatchPair*)(const MH_CONST BatchPair*)p;
+}
+
 // The last slice of a split tile to arrive (the partial tiles hold pm x pn
 // elements per tile and slice, pm = min(M, BM), pn = min(N, BN)) sums the
 // slices in slice order and writes C, so the result does not depend on which
@@ -77,10 +87,19 @@ __device__ __forceinline__ void split_tile_fixup(const BatchPair& pr, int bz, in
   }
 }
 
+// SEP: K is whole K-tiles, each addressed from one base per tile.  Looking every
+// element's k up made each K-tile's loads wait for its table entries, and the
+// pair's descriptor went through vector loads at every use.  With scalar bases,
+// 32-bit thread offsets and the descriptor in scalar registers the persistent
+// kernel takes 704 us in place of 978 for the 54 such pairs of a 256-pair batch
+// (complex FP64, 433 us of products), the split kernel 75 in place of 98, and
+// batches that are mostly such pairs gain more (89 pairs to rank 19: 575 to
+// 387 us).  Bound by the two workgroups a CU holds at 256 registers: 64 x 64
+// tiles of 2 to 8 K-tiles spend a third of their time in first loads and stores.
 // DB: double-buffered LDS (one barrier per K-tile, the gather of K-tile
 // t + 1 in flight while t is multiplied); the 64 x 64 shape uses it, the
 // skinny shapes keep one buffer so every shape fits the same LDS budget.
-template <typename T, bool CP, bool G3, int BM, int BN, int WM, int WN, bool DB, bool SPLIT>
+template <typename T, bool CP, bool G3, int BM, int BN, int WM, int WN, bool DB, bool SPLIT, bool SEP>
 __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, int tn, int slice, T* lds,
                                            int* s_flag) {
   using MM = Mma<T>;
@@ -100,9 +119,10 @@ __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, 
   const int M = pr.M, N = pr.N, K = pr.K;
   // this item's K range: the whole of K, or one slice of a split pair
   const int kbeg = slice * pr.kchunk, kend = min(K, kbeg + pr.kchunk);
-  const int64_t offA0 = pr.bA[bz], offB0 = pr.bB[bz], offC0 = pr.bC[bz];
+  const int64_t offA0 = uniform_offset(pr.bA, bz), offB0 = uniform_offset(pr.bB, bz), offC0 = uniform_offset(pr.bC, bz);
 
   int a_mm[NEA], a_kk[NEA], b_nn[NEB], b_kk[NEB];
+  asm volatile("" ::"i"(BM * 2 + SEP));  // keeps the variants apart
   bool a_ok[NEA], b_ok[NEB];
   int64_t a_row[NEA], b_col[NEB];
 #pragma unroll
@@ -116,8 +136,10 @@ __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, 
       a_kk[i] = e / BM;
     }
     const int m = m0 + a_mm[i];
-    a_ok[i] = m < M;
-    a_row[i] = pr.rowA[a_ok[i] ? m : M - 1] + offA0;
+    if constexpr (!SEP) {
+      a_ok[i] = m < M;
+      a_row[i] = pr.rowA[a_ok[i] ? m : M - 1] + offA0;
+    }
     a_mm[i] ^= a_kk[i];  // from here on: the swizzled LDS column
   }
 #pragma unroll
@@ -131,8 +153,10 @@ __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, 
       b_kk[i] = e / BN;
     }
     const int n = n0 + b_nn[i];
-    b_ok[i] = n < N;
-    b_col[i] = pr.colB[b_ok[i] ? n : N - 1] + offB0;
+    if constexpr (!SEP) {
+      b_ok[i] = n < N;
+      b_col[i] = pr.colB[b_ok[i] ? n : N - 1] + offB0;
+    }
     b_nn[i] ^= b_kk[i];
   }
   // this lane's MFMA reads at K step ks (rows k = 4 ks + (lane >> 4)): the
@@ -216,14 +240,62 @@ __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, 
 
   // K-tiles kt0 .. kt1 - 1 (kbeg is a multiple of BK)
   const int kt0 = kbeg / BK, kt1 = (kend + BK - 1) / BK;
-  if (kt0 < kt1) MH_GATHER(kt0);
+  // SEP (K a multiple of BK): each K-tile from its base and this thread's 32-bit
+  // byte offsets.  Rows and columns outside M and N are clamped: their products
+  // reach no output.
+  constexpr int ES = (int)sizeof(T) * PL;
+  uint32_t va[NEA], vb[NEB];
+  const char* const bA = (const char*)pr.A + (offA0 + pr.minA) * ES;
+  const char* const bB = (const char*)pr.B + (offB0 + pr.minB) * ES;
+  if constexpr (SEP) {
+    uint32_t im[NEA], in[NEB], ia[NEA], ib[NEB];
+    int64_t om[NEA], on[NEB], ka[NEA], kb[NEB];
+#pragma unroll
+    for (int i = 0; i < NEA; ++i) {
+      im[i] = (uint32_t)min(m0 + (a_mm[i] ^ a_kk[i]), M - 1);
+      ia[i] = (uint32_t)(kbeg + a_kk[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) {
+      in[i] = (uint32_t)min(n0 + (b_nn[i] ^ b_kk[i]), N - 1);
+      ib[i] = (uint32_t)(kbeg + b_kk[i]);
+    }
+    load_offsets<NEA>(pr.rowA, im, om);
+    load_offsets<NEB>(pr.colB, in, on);
+    load_offsets<NEA>(pr.kA, ia, ka);
+    load_offsets<NEB>(pr.kB, ib, kb);
+    const int64_t a0 = uniform_offset(pr.kA, kbeg) + pr.minA, b0 = uniform_offset(pr.kB, kbeg) + pr.minB;
+#pragma unroll
+    for (int i = 0; i < NEA; ++i) va[i] = (uint32_t)((om[i] + ka[i] - a0) * ES);
+#pragma unroll
+    for (int i = 0; i < NEB; ++i) vb[i] = (uint32_t)((on[i] + kb[i] - b0) * ES);
+  }
+  auto gather = [&](int kt) {
+    if constexpr (!SEP) {
+      MH_GATHER(kt);
+    } else {
+      const char* const ga = bA + uniform_offset(pr.kA, kt * BK) * ES;
+      const char* const gb = bB + uniform_offset(pr.kB, kt * BK) * ES;
+#pragma unroll
+      for (int i = 0; i < NEA; ++i) {
+        asm volatile("" : "+v"(va[i]));  // keeps the 32-bit offset a register of its own
+        ra[i] = load_elem<T, CP>(ga + va[i], 0);
+      }
+#pragma unroll
+      for (int i = 0; i < NEB; ++i) {
+        asm volatile("" : "+v"(vb[i]));
+        rb[i] = load_elem<T, CP>(gb + vb[i], 0);
+      }
+    }
+  };
+  if (kt0 < kt1) gather(kt0);
   if constexpr (DB) {
     __syncthreads();  // the previous tile's readers of buffer 0 are done
     if (kt0 < kt1) MH_STASH(0);
     __syncthreads();
     for (int kt = kt0; kt < kt1; ++kt) {
       const int cur = (kt - kt0) & 1;
-      if (kt + 1 < kt1) MH_GATHER(kt + 1);
+      if (kt + 1 < kt1) gather(kt + 1);
       // FP64: the MFMA section at raised wave priority, as in the plain tiles
       if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
       MH_COMPUTE(cur);
@@ -236,7 +308,7 @@ __device__ __forceinline__ void batch_tile(const BatchPair& pr, int bz, int tm, 
       __syncthreads();  // earlier readers of the LDS tile are done
       MH_STASH(0);
       __syncthreads();
-      if (kt + 1 < kt1) MH_GATHER(kt + 1);
+      if (kt + 1 < kt1) gather(kt + 1);
       if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
       MH_COMPUTE(0);
       if constexpr (sizeof(T) == 8) __builtin_amdgcn_s_setprio(0);
@@ -330,18 +402,21 @@ __global__ __launch_bounds__(NT, kBatchWgPerCu) void batch_kernel(BatchArgs a) {
     const int64_t it = *s_item;
     __syncthreads();  // every thread holds the item before thread 0 fetches the next
     if (it < 0) break;
-    const int2 w = a.items[it];
-    const BatchPair& pr = a.pairs[w.x];
+    const int2 w = uniform_item(a.items + it);
+    const BatchPair& pr = uniform_pair(a.pairs + w.x);
     const int per_batch = pr.tiles_m * pr.tiles_n;
     // w.y = tile * ksplit + slice
     const int t = w.y / pr.ksplit, slice = w.y - t * pr.ksplit;
     const int bz = t / per_batch;
     const int r = t - bz * per_batch;
     const int tm = r / pr.tiles_n, tn = r - tm * pr.tiles_n;
-    switch (pr.tile) {
-      case 0: batch_tile<T, CP, G3, 64, 64, 2, 2, true, false>(pr, bz, tm, tn, slice, lds, s_item); break;
-      case 1: batch_tile<T, CP, G3, 32, 128, 1, 4, false, false>(pr, bz, tm, tn, slice, lds, s_item); break;
-      default: batch_tile<T, CP, G3, 128, 32, 4, 1, false, false>(pr, bz, tm, tn, slice, lds, s_item); break;
+    switch (pr.tile * 2 + pr.ktile16) {
+      case 0: batch_tile<T, CP, G3, 64, 64, 2, 2, true, false, false>(pr, bz, tm, tn, slice, lds, s_item); break;
+      case 1: batch_tile<T, CP, G3, 64, 64, 2, 2, true, false, true>(pr, bz, tm, tn, slice, lds, s_item); break;
+      case 2: batch_tile<T, CP, G3, 32, 128, 1, 4, false, false, false>(pr, bz, tm, tn, slice, lds, s_item); break;
+      case 3: batch_tile<T, CP, G3, 32, 128, 1, 4, false, false, true>(pr, bz, tm, tn, slice, lds, s_item); break;
+      case 4: batch_tile<T, CP, G3, 128, 32, 4, 1, false, false, false>(pr, bz, tm, tn, slice, lds, s_item); break;
+      default: batch_tile<T, CP, G3, 128, 32, 4, 1, false, false, true>(pr, bz, tm, tn, slice, lds, s_item); break;
     }
   }
 }
@@ -356,17 +431,20 @@ __global__ __launch_bounds__(NT, kBatchWgPerCu) void split_kernel(BatchArgs a) {
   T* lds = reinterpret_cast<T*>(smem_raw);
   int* s_flag = reinterpret_cast<int*>(smem_raw + a.item_off);
   for (int64_t it = blockIdx.x; it < a.nitems; it += gridDim.x) {
-    const int2 w = a.items[it];
-    const BatchPair& pr = a.pairs[w.x];
+    const int2 w = uniform_item(a.items + it);
+    const BatchPair& pr = uniform_pair(a.pairs + w.x);
     const int per_batch = pr.tiles_m * pr.tiles_n;
     const int t = w.y / pr.ksplit, slice = w.y - t * pr.ksplit;
     const int bz = t / per_batch;
     const int r = t - bz * per_batch;
     const int tm = r / pr.tiles_n, tn = r - tm * pr.tiles_n;
-    switch (pr.tile) {
-      case 0: batch_tile<T, CP, G3, 64, 64, 2, 2, true, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
-      case 1: batch_tile<T, CP, G3, 32, 128, 1, 4, false, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
-      default: batch_tile<T, CP, G3, 128, 32, 4, 1, false, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
+    switch (pr.tile * 2 + pr.ktile16) {
+      case 0: batch_tile<T, CP, G3, 64, 64, 2, 2, true, true, false>(pr, bz, tm, tn, slice, lds, s_flag); break;
+      case 1: batch_tile<T, CP, G3, 64, 64, 2, 2, true, true, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
+      case 2: batch_tile<T, CP, G3, 32, 128, 1, 4, false, true, false>(pr, bz, tm, tn, slice, lds, s_flag); break;
+      case 3: batch_tile<T, CP, G3, 32, 128, 1, 4, false, true, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
+      case 4: batch_tile<T, CP, G3, 128, 32, 4, 1, false, true, false>(pr, bz, tm, tn, slice, lds, s_flag); break;
+      default: batch_tile<T, CP, G3, 128, 32, 4, 1, false, true, true>(pr, bz, tm, tn, slice, lds, s_flag); break;
     }
   }
 }

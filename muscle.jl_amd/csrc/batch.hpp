@@ -25,6 +25,9 @@ struct BatchPair {
   // split K: ksplit slices of kchunk elements per output tile (1 and K when
   // not split); the slices' partial tiles and the tiles' arrival counters
   int32_t ksplit, kchunk;
+  // K is whole K-tiles of 16, each addressed from one base (GemmArgs::ktile16)
+  int32_t ktile16, pad;
+  int64_t minA, minB;
   void* partial;
   int32_t* tilecnt;
   OffTab rowA, kA, kB, colB, rowC, colC, bA, bB, bC;
@@ -217,6 +220,8 @@ struct PlannedPair {
   void* c = nullptr;
   const int64_t* dtab = nullptr;  // device tables of this pair; null: the batch's own table region
   const std::vector<int64_t>* htab = nullptr;  // the host copy its TabRefs index
+  bool ktile16 = false;           // and the lowest offsets (BatchPair)
+  int64_t min_a = 0, min_b = 0;
   bool solo = false;              // runs as a single-contraction launch, not in the work list
   // bits: the power-of-two kernel takes the pair in any launch where its route
   // is shallow or skinny; bits_only: it has no other route, and no tables

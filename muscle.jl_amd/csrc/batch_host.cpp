@@ -139,6 +139,12 @@ void plan_pair(const Handle& h, PlannedPair& L, std::vector<int64_t>& htab, int 
   const std::vector<Dim>* cls[4] = {&d.m, &d.n, &d.k, &d.batch};
   for (int t = 0; t < 9 && !L.bits_only; ++t) L.t[t] = add_table(htab, *cls[T3[t][0]], T3[t][1], single_max);
   L.htab = &htab;
+  if (!L.bits_only && d.K > kShallowK) {
+    const KTiles kt = k_tiles(d);
+    L.ktile16 = kt.ktile16 && d.K % 16 == 0;
+    L.min_a = kt.min_a;
+    L.min_b = kt.min_b;
+  }
   if (tile < 0 || tile >= MUSCLE_HIP_TILE_COUNT) {
     const int tc = h.tune[tuning_class(d.M, d.N)];
     tile = tc >= 0 ? tc : default_tile(d.M, d.N);
@@ -447,6 +453,9 @@ void place_batch(Batch& B, const std::vector<const PlannedPair*>& lw, char* base
     P.a_kmajor = L.a_kmajor;
     P.b_kmajor = L.b_kmajor;
     P.c_mfast = L.c_mfast;
+    P.ktile16 = L.ktile16;
+    P.minA = L.min_a;
+    P.minB = L.min_b;
     P.c_stream = c_stream_of(L.d);
     P.ksplit = B.ksplit.empty() ? 1 : B.ksplit[(size_t)i];
     P.kchunk = B.kchunk.empty() || B.kchunk[(size_t)i] == 0 ? P.K : B.kchunk[(size_t)i];

@@ -38,11 +38,6 @@ namespace {
 
 constexpr int NT = 1 << kBitThread;
 
-#if defined(__HIP_DEVICE_COMPILE__)
-#define MH_CONST __attribute__((address_space(4)))
-#else
-#define MH_CONST
-#endif
 typedef const MH_CONST BitDesc* DescPtr;  // read through the scalar cache
 
 // The other vector-FMA kernels' sums in their order: a contraction's result does

@@ -1,6 +1,7 @@
 // Device-side element types and arithmetic helpers.
 #pragma once
 
+#include "kernels.hpp"
 #include <hip/hip_runtime.h>
 
 namespace mh {
@@ -97,6 +98,41 @@ __device__ inline void gemm_tile_coords(int L, int nwg, int tiles_m, int tiles_n
   const int r = L - g * per_group;
   tm = first_m + r % gsize;
   tn = r / gsize;
+}
+
+// Entries of one offset table, with one test of its form for all of them.
+template <int N>
+__device__ __forceinline__ void load_offsets(const OffTab& t, const uint32_t* i, int64_t* out) {
+  typedef const MH_GLOBAL int64_t* gp;
+  const gp lo = gptr<int64_t>(t.lo), hi = gptr<int64_t>(t.hi);
+  if (t.single) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] = lo[i[e] + t.base];
+  } else {
+    int64_t h[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const uint32_t x = i[e] + t.base, q = t.div.div(x);
+      out[e] = lo[x - q * t.div.d];
+      h[e] = hi[q];
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) out[e] += h[e];
+  }
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MH_CONST __attribute__((address_space(4)))
+#else
+#define MH_CONST
+#endif
+// The entry at a wave-uniform index, read through the scalar cache.
+__device__ __forceinline__ int64_t uniform_offset(const OffTab& t, uint32_t i) {
+  typedef const MH_CONST int64_t* cp;
+  const cp lo = (cp)t.lo, hi = (cp)t.hi;
+  i += t.base;
+  if (t.single) return lo[i];
+  const uint32_t q = t.div.div(i);
+  return lo[i - q * t.div.d] + hi[q];
 }
 
 }  // namespace mh

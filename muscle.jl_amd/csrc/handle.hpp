@@ -124,6 +124,13 @@ extern thread_local std::string g_last_error;
 std::unique_ptr<Plan> build_contraction_plan(const ContractionDesc& d, int precision);
 // Split-K slices of a tile-GEMM plan (one slice for plans of other kinds).
 void plan_gemm_ksplit(Plan& p);
+// Whether K-tiles of 8 (16) have a common base (GemmArgs::ktile8), and the
+// lowest offsets of a K-tile's rows and columns.
+struct KTiles {
+  bool ktile8, ktile16;
+  int64_t min_a, min_b;
+};
+KTiles k_tiles(const ContractionDesc& d);
 void upload_tables(Plan& p, hipStream_t s);
 // Enqueues one planned contraction on h.stream.  Its workspace is the
 // handle's (grown as needed), or `ws` of `ws_size` bytes when given (no
