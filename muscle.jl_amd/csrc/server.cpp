@@ -198,7 +198,7 @@ struct Server {
   // the single-precision jobs' stream, plans and workspace: a tick's launches
   // are short chains of few workgroups, so two element types one after the
   // other leave most of the GPU idle (24 jobs of both, 20 to 300 contractions
-  // each: 8 ms of launches in a row of 10 ms, side by side 5)
+  // each: from the first launch to the last 10.0 ms, side by side 8.0)
   Handle hs;
   int mode = 0;
   int max_active = 64;
