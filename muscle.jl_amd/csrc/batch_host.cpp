@@ -278,7 +278,8 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
         for (int64_t t = 0; t < items; ++t) xq[x].push_back(make_int2((int)i, (int)t));
         xload[x] += cost * (double)items;
       }
-    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small) && small.nchunk <= kBitSmallChunks))) {
+    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small) &&
+                                         small.nchunk <= kBitSmallChunks))) {
       const int32_t x = (int32_t)B.hbits.size();
       B.bit_index[(size_t)i] = x;
       B.hbits.push_back(L.bits ? L.bit : small);
