@@ -66,7 +66,7 @@ bool plan_bits(const ContractionDesc& d, BitDesc& out) {
   if (!bits_of(d.m, M, c) || !bits_of(d.n, N, c) || !bits_of(d.batch, BATCH, c) || !bits_of(d.k, BATCH, k)) return false;
   const int nc = (int)c.size(), nk = (int)k.size();
   if (nc < kBitTile || nc - kBitTile > kBitOuter - 2 || nk > kBitChunk) return false;
-  // every offset fits 32 bits
+  // every element offset fits 32 bits
   for (int w = 0; w < 3; ++w) {
     int64_t span = 1;
     for (auto& b : c) span += b.s[w];
@@ -174,6 +174,14 @@ bool plan_bits(const ContractionDesc& d, BitDesc& out) {
   }
   out.nl = plan_gather(gl, out.gL, out.gLl, out.iL, out.iLl, kBitLongIt);
   out.ns = plan_gather(gs, out.gS, out.gSl, out.iS, out.iSl, kBitShortIt);
+  // a thread's own byte offsets are 32-bit registers: an operand that spreads a
+  // tile over 4 GiB or more (a gate on a state of 2^30 ComplexF64 elements, its
+  // new sites last) is left to the kernels with 64-bit offsets
+  for (const uint32_t* s : {out.tC, out.gL, out.gS}) {
+    uint64_t most = 0;
+    for (int j = 0; j < kBitThread; ++j) most += s[j];
+    if (most * (uint64_t)es >= uint64_t(1) << 32) return false;
+  }
   out.kc = 1 << kcb;
   out.nchunk = 1 << (nk - kcb);
   uint32_t cl = 0, cs = 0;  // the lower bits' strides together

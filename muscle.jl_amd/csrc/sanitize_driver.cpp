@@ -433,6 +433,100 @@ void check_bits(std::mt19937_64& rng) {
   std::printf("power-of-two kernel: %d plans run on the host, %d with K chunks\n", planned, chunked);
 }
 
+// Operands too large to hold here, by their strides alone: wherever the
+// power-of-two kernel takes a contraction, the byte offsets that its threads
+// form in 32 bits have the value they have in 64, and its steps from tile to
+// tile land where the tile's number says.
+void check_bits_offsets(std::mt19937_64& rng) {
+  int planned = 0, large = 0;
+  auto check = [&](const muscle_hip_tensor_t& tc, const muscle_hip_tensor_t& ta, const muscle_hip_tensor_t& tb,
+                   int64_t detail) {
+    mh::BitDesc q;
+    const mh::ContractionDesc d = mh::lower_binary(tc, ta, tb);
+    if (!mh::plan_bits(d, q)) return false;
+    ++planned;
+    const uint32_t ES = (uint32_t)esize(tc.dtype);
+    bool same = true, steps = true;
+    for (uint32_t tid = 0; tid < (1u << mh::kBitThread); ++tid)
+      for (const uint32_t* s : {q.tC, q.gL, q.gS}) {
+        uint32_t v = 0;
+        uint64_t exact = 0;
+        for (int j = 0; j < mh::kBitThread; ++j)
+          if (tid >> j & 1) {
+            v += s[j];
+            exact += s[j];
+          }
+        same = same && (uint64_t)(uint32_t)(v * ES) == exact * ES;
+      }
+    const uint32_t* o[3] = {q.oL, q.oS, q.oC};
+    const uint32_t* st[3] = {q.sL, q.sS, q.sC};
+    for (int w = 0; w < 3; ++w) {
+      auto at = [&](uint32_t t) {
+        uint32_t x = 0;
+        for (int j = 0; j < mh::kBitOuter; ++j)
+          if (t >> j & 1) x += o[w][j];
+        return x;
+      };
+      for (uint32_t t0 : {0u, (uint32_t)(q.tiles - q.run)})
+        for (uint32_t t = t0; t + 1 < t0 + (uint32_t)q.run; ++t)
+          steps = steps && at(t) + st[w][__builtin_ctz(t + 1)] == at(t + 1);
+    }
+    large += q.run == 8;
+    expect(same, "power-of-two plan: a thread's byte offset beyond 32 bits", detail);
+    expect(steps, "power-of-two plan: tile steps of a full run", detail);
+    return true;
+  };
+  // gates on states of up to 2^32 elements, the new sites last in the output
+  for (int dt = 0; dt < 4; ++dt)
+    for (int sites = 26; sites <= 32; ++sites)
+      for (int it = 0; it < 24; ++it) {
+        const int qubits = 1 + it % 3;
+        std::vector<int32_t> all((size_t)sites);
+        for (int i = 0; i < sites; ++i) all[(size_t)i] = i + 1;
+        std::shuffle(all.begin(), all.end(), rng);
+        Operand st, g, c;
+        auto mode = [&](Operand& x, int32_t l) {
+          x.modes.push_back(l);
+          x.ext.push_back(2);
+          x.strides.push_back(int64_t(1) << (x.modes.size() - 1));
+        };
+        for (int l = 1; l <= sites; ++l) {
+          mode(st, l);
+          if (std::find(all.begin(), all.begin() + qubits, l) == all.begin() + qubits) mode(c, l);
+        }
+        for (int i = 0; i < qubits; ++i) mode(g, sites + 1 + i);
+        for (int i = 0; i < qubits; ++i) mode(g, all[(size_t)i]);
+        for (int i = 0; i < qubits; ++i) mode(c, sites + 1 + i);
+        const bool ok = check(c.desc(dt, (void*)256), st.desc(dt, (void*)256), g.desc(dt, (void*)256), sites * 100 + it);
+        expect(ok || sites >= 29 || qubits == 1, "a gate on a state of 2 to 4 GB stays with the power-of-two kernel",
+               sites * 100 + it);
+      }
+  // strided views: a wide gap above one mode of one operand
+  for (int it = 0; it < 600; ++it) {
+    std::vector<int64_t> extent(1, 1);
+    std::vector<int32_t> la, lb, lc;
+    const int bits = 11 + (int)(rng() % 4), kbits = 1 + (int)(rng() % 4);
+    for (int i = 0; i < bits + kbits; ++i) {
+      extent.push_back(2);
+      const int32_t l = (int32_t)extent.size() - 1;
+      if (i < bits) lc.push_back(l);
+      const int to = (int)(rng() % 2);
+      if (i >= bits || to == 0) la.push_back(l);
+      if (i >= bits || to == 1) lb.push_back(l);
+    }
+    Operand x[3] = {make_operand(la, extent, rng), make_operand(lb, extent, rng), make_operand(lc, extent, rng)};
+    Operand& y = x[rng() % 3];
+    if (y.strides.empty()) continue;
+    const size_t from = rng() % y.strides.size();
+    const int shift = 10 + (int)(rng() % 14);
+    for (size_t i = from; i < y.strides.size(); ++i) y.strides[i] <<= shift;
+    const int dt = (int)(rng() % 4);
+    check(x[2].desc(dt, (void*)256), x[0].desc(dt, (void*)256), x[1].desc(dt, (void*)256), it);
+  }
+  expect(planned > 300 && large > 100, "power-of-two plans of large operands", planned);
+  std::printf("power-of-two kernel: offsets of %d plans of large operands checked\n", planned);
+}
+
 bool is_cplx(int dt) { return dt == MUSCLE_HIP_C32 || dt == MUSCLE_HIP_C64; }
 
 std::vector<char> encode(const std::vector<cd>& v, int dt) {
@@ -686,6 +780,8 @@ int main(int argc, char** argv) {
   std::mt19937_64 rng_k(20261204);
   check_ktiles(rng_k);
   check_bits(rng_k);
+  std::mt19937_64 rng_o(20261205);
+  check_bits_offsets(rng_o);
   if (argc > 1 && std::strcmp(argv[1], "--gpu") == 0) check_gpu(rng);
   std::printf("%s: %d failures\n", g_failures ? "FAILED" : "ok", g_failures);
   return g_failures ? 1 : 0;
