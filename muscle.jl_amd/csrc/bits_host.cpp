@@ -21,10 +21,10 @@ struct Bit {
 };
 
 // The bits of a dim list, fastest first; false unless every extent is a power
-// of two and every stride is usable (nonnegative).
+// of two (0, an empty sum, is none) and every stride is usable (nonnegative).
 bool bits_of(const std::vector<Dim>& v, int cls, std::vector<Bit>& out) {
   for (auto& x : v) {
-    if (x.extent & (x.extent - 1)) return false;
+    if (x.extent < 1 || (x.extent & (x.extent - 1))) return false;
     for (int w = 0; w < 3; ++w)
       if (x.s[w] < 0) return false;
     for (int64_t e = 1; e < x.extent; e <<= 1) out.push_back(Bit{cls, {x.s[0] * e, x.s[1] * e, x.s[2] * e}});

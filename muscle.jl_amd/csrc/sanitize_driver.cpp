@@ -527,6 +527,33 @@ void check_bits_offsets(std::mt19937_64& rng) {
   std::printf("power-of-two kernel: offsets of %d plans of large operands checked\n", planned);
 }
 
+// A contracted mode without elements (M = 2^16, N = 4 and M = 2^18, N = 1 are
+// large enough for the power-of-two kernel otherwise): the sum is empty, and
+// neither operand has an element to read.
+void check_bits_empty() {
+  int others = 0;
+  for (int dt = 0; dt < 4; ++dt)
+    for (int64_t n : {1, 4})
+      for (int64_t k2 : {1, 2})
+        for (int64_t k : {0, 2}) {
+          const int64_t m = n == 1 ? 1 << 18 : 1 << 16;
+          Operand a{{1, 3, 4}, {m, k, k2}, {1, m, m * 2}}, b{{3, 4, 2}, {k, k2, n}, {1, 2, 2 * k2}},
+              c{{1, 2}, {m, n}, {1, m}};
+          const muscle_hip_tensor_t tc = c.desc(dt, (void*)256), ta = a.desc(dt, k ? (void*)256 : nullptr),
+                                    tb = b.desc(dt, k ? (void*)256 : nullptr);
+          const mh::ContractionDesc d = mh::lower_binary(tc, ta, tb);
+          mh::BitDesc q;
+          const int kind = mh::build_contraction_plan(d, MUSCLE_HIP_PRECISION_NATIVE)->kind;
+          if (k == 0) {
+            expect(!mh::plan_bits(d, q), "power-of-two plan of an empty sum", dt * 100 + n * 10 + k2);
+            expect(kind == mh::Plan::REDUCE, "kernel of an empty sum", kind);
+          } else if (kind == mh::Plan::BITS) {
+            ++others;
+          }
+        }
+  expect(others > 0, "the same sizes with elements to sum", others);
+}
+
 bool is_cplx(int dt) { return dt == MUSCLE_HIP_C32 || dt == MUSCLE_HIP_C64; }
 
 std::vector<char> encode(const std::vector<cd>& v, int dt) {
@@ -782,6 +809,7 @@ int main(int argc, char** argv) {
   check_bits(rng_k);
   std::mt19937_64 rng_o(20261205);
   check_bits_offsets(rng_o);
+  check_bits_empty();
   if (argc > 1 && std::strcmp(argv[1], "--gpu") == 0) check_gpu(rng);
   std::printf("%s: %d failures\n", g_failures ? "FAILED" : "ok", g_failures);
   return g_failures ? 1 : 0;

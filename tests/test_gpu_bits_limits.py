@@ -48,3 +48,26 @@ def test_tile_over_4_gib(T, wide, batched):
     assert rel_err(c.parent().cpu().numpy().reshape(ref.shape), ref) <= TOL[T]
     # nothing else in the output's storage was written
     assert int(torch.count_nonzero(flat)) == int(np.count_nonzero(c.parent().cpu().numpy()))
+
+
+@pytest.mark.parametrize("batched", [False, True], ids=["plain", "batch"])
+@pytest.mark.parametrize("shape", [(1 << 16, 4), (1 << 18, 1), (1 << 10, 1 << 10)], ids=str)
+@pytest.mark.parametrize("T", [np.complex128, np.float32])
+def test_empty_sum(T, shape, batched):
+    """Sizes that the power-of-two kernel would take, but for a contracted mode without elements: zeros,
+    in every element of an output that starts as NaN."""
+    m, n = shape
+    t = lambda size, labels: muscle.Tensor(  # noqa: E731
+        torch.full(size, float("nan"), dtype=NP2TORCH[T], device="cuda"), list(labels))
+    a, b, c = t((m, 0, 2), "ikl"), t((0, 2, n), "klj"), t((m, n), "ij")
+    if batched:  # beside a pair that the power-of-two kernel does take
+        x = torch.ones(2, 1 << 5, dtype=NP2TORCH[T], device="cuda")
+        y = torch.ones(1 << 15, 2, dtype=NP2TORCH[T], device="cuda")
+        z = t((1 << 15, 1 << 5), "ji")
+        ContractionBatch([(c, a, b), (z, muscle.Tensor(x, list("ki")), muscle.Tensor(y, list("jk")))]).run()
+    else:
+        muscle.binary_einsum_(c, a, b)
+    torch.cuda.synchronize()
+    assert torch.equal(c.parent(), torch.zeros_like(c.parent()))
+    if batched:
+        assert torch.equal(z.parent(), torch.full_like(z.parent(), 2))
