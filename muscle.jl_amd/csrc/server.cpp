@@ -574,20 +574,21 @@ void Server::loop() {
           continue;
         }
       }
-      for (auto& j : admitted)
-        if (j->dtab_bytes)
-          MH_HIP_CHECK(hipMemcpyAsync(j->dtab, j->htab.data(), j->htab.size() * sizeof(int64_t),
-                                      hipMemcpyHostToDevice, lane(lane_of(j->dtype)).stream));
       if (mode == 1) {
         std::shared_ptr<Job> j;
         {
           std::lock_guard<std::mutex> lk(mu);
           if (!active.empty()) j = active.front();
         }
-        if (j) run_serial(*j);
+        if (j) run_serial(*j);  // its plans bring their own tables
         cv_done.notify_all();
         continue;
       }
+      // the batched contractions' tables, ahead of the job's launches on its stream
+      for (auto& j : admitted)
+        if (j->dtab_bytes)
+          MH_HIP_CHECK(hipMemcpyAsync(j->dtab, j->htab.data(), j->htab.size() * sizeof(int64_t),
+                                      hipMemcpyHostToDevice, lane(lane_of(j->dtype)).stream));
       progress |= complete_ticks(false);
       progress |= launch_tick();
       if (!progress) {
