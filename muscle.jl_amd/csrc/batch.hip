@@ -725,13 +725,7 @@ __global__ __launch_bounds__(SNT, CP ? 6 : 4) void shallow_one_kernel(ShallowArg
 // complex product (a from A, b from B), so a pair's result does not depend on
 // the orientation or on what else is in the batch.
 constexpr int KNT = 512;   // threads per workgroup
-// short-side operand elements staged per chunk.  In FP64 this leaves one
-// workgroup per CU: where a line of the long operand runs along K, a workgroup's
-// threads hold 64 KB of lines between one k and the next, and those of two or
-// three workgroups on 32 CUs no longer fit the XCD's L2 (the skinny pairs of a
-// 256-pair batch: 920 us with 2048, 817 with 4096; 16 more registers for two
-// workgroups and loads of 4 k together 1022, for one 869).
-constexpr int KSB = 4096;
+constexpr int KSB = 2048;  // short-side operand elements staged per chunk
 constexpr int KOFF_S = 2 * kSkinnyMaxK, KOFF_C = KOFF_S + kSkinnyMaxS, KOFF_N = KOFF_C + kSkinnyMaxS;
 
 // SM: the short side is M (A is the short operand, B the long one, C's long
