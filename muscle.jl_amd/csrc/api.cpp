@@ -214,19 +214,40 @@ bool precision_plain(const ContractionDesc& d, int precision) {
   return precision == MUSCLE_HIP_PRECISION_NATIVE || !is_double(d.dt[2]) || d.M < 16 || d.N < 16 || d.K < 16;
 }
 
-// Contractions the power-of-two kernel is for, by what the other kernels
-// measured on the same pairs (complex FP64, us, other / power-of-two).  A sum
-// too short for the matrix tiles: 2^2 x 2^20 x 2^2 145 / 25, 2^12 x 2^12 x 2 167
-// / 61, but 2^8 x 2^8 x 2 x 2 (64 tiles) 4.2 / 4.7: from 128 tiles on.  Both
-// sides 32 or more: K = 8, 2^6 x 2^6 8.1 / 5.2, 2^12 x 2^12 85 / 57; K = 16,
-// 2^12 x 2^12 86 / 77, with kept modes 2^16 x 2^6 (x 4) 90 / 96: only without
-// them.  A short side and K = 16 to 128: 2^4 x 2^18 x 2^6 184 / 98, 2^3 x 2^18 x
-// 2^7 307 / 242, 2^4 x 2^14 x 2^6 x 2 (256 tiles) 25 / 39, K = 256 from 1.7
-// times faster to 1.3 times slower: from 512 tiles and up to K = 128.
-bool bits_wanted(const ContractionDesc& d) {
+// Contractions the power-of-two kernel is for, and its plan.  The lines come from
+// 5888 contractions in all four types, three mode orders or more each (time over
+// the reduction kernel's or the tile GEMM's, least / median / most):
+//   a sum too short for the matrix tiles, in one chunk: 0.06 / 0.4 / 1.1 from 128
+//     tiles on, in 2 or 4 chunks from 256 (128: 0.6 / 1.0 / 1.6), in 8 from 512;
+//   both sides 32 or more, K = 8: 0.4 / 0.8 / 1.3; K = 16: 0.6 / 1.1 / 1.5, with 1024 to
+//     4095 tiles (the GEMM's fill the chip evenly) or 4 chunks up to 1.8, with kept
+//     modes 1.1;
+//   a short side and K = 16 to 128, 512 tiles or more (256: 25 us / 39): complex FP64
+//     0.2 / 0.75 / 1.5 (GEMM before its loop was reworked: 0.2 / 0.4 / 0.9).  The others'
+//     matrix tiles are faster: 4 bytes 0.2 / 0.5 / 0.8 to 8 chunks, beyond with a side
+//     of 4 or 8 up to 1.5; 8 bytes to 16 chunks 0.3 / 0.6 / 1.2, 32 where no line of the
+//     long operand runs along K or all of it does; a side of 16 (the tiles pad it
+//     only to 32 or 64) 4 chunks 0.55 / 0.75 / 1.3, more up to 2.3;
+//   a side of 1 or 2 whose long operand runs along K but for 32 bytes (over the
+//     side) of each line: a chunk fetches part of every line, 1.2 to 5.8.
+bool bits_for(const ContractionDesc& d, BitDesc& q) {
+  const int64_t side = std::min(d.M, d.N), es = (int64_t)dtype_size(d.dt[2]);
   const double tiles = (double)d.M * (double)d.N * (double)d.B / (1 << kBitTile);
-  if (std::min(d.M, d.N) >= 32) return d.K < 8 ? tiles >= 128 : d.K == 8 || (d.K == 16 && d.B == 1);
-  return d.K <= 8 ? tiles >= 128 : std::min(d.M, d.N) <= 16 && d.K <= 128 && tiles >= 512;
+  if (side >= 32) {
+    if (d.K < 8 ? tiles < 128 : d.K > 16 || (d.K == 16 && d.B > 1)) return false;
+    return plan_bits(d, q) && (d.K <= 8 || (q.nchunk <= 2 && (tiles < 1024 || tiles >= 4096)));
+  }
+  if (d.K <= 8 ? tiles < 128 : side > 16 || d.K > 128 || tiles < 512) return false;
+  if (!plan_bits(d, q)) return false;
+  const int nc = q.nchunk;
+  if (side <= 2 && nc > 2 && side * (128 >> q.line_k) <= 32) return false;
+  if (d.K <= 8) return tiles >= (nc == 1 ? 128 : nc <= 4 ? 256 : 512);
+  if (es == 16) return true;
+  const bool whole_lines = (es << q.line_k) == 128;
+  if (side == 16) return nc <= (whole_lines && es == 8 ? 8 : tiles >= 1024 ? 4 : 2);
+  if (whole_lines && es == 8) return true;
+  if (side == 8 ? es == 4 || tiles < 1024 : es == 4 && side == 4 && q.line_split) return nc <= 8;
+  return nc <= (side <= 2 || q.line_k == 0 ? 32 : 16);
 }
 
 }  // namespace
@@ -242,7 +263,7 @@ std::unique_ptr<Plan> build_contraction_plan(const ContractionDesc& d, int preci
   }
   // Little work per output and power-of-two extents throughout: tiles of C in
   // address order.
-  if (d.has_b && precision_plain(d, precision) && bits_wanted(d) && plan_bits(d, p->bits)) {
+  if (d.has_b && precision_plain(d, precision) && bits_for(d, p->bits)) {
     p->kind = Plan::BITS;
     return p;
   }

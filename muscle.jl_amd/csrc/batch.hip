@@ -725,7 +725,11 @@ __global__ __launch_bounds__(SNT, CP ? 6 : 4) void shallow_one_kernel(ShallowArg
 // complex product (a from A, b from B), so a pair's result does not depend on
 // the orientation or on what else is in the batch.
 constexpr int KNT = 512;   // threads per workgroup
-constexpr int KSB = 2048;  // short-side operand elements staged per chunk
+// short-side operand elements staged per chunk.  With 4096 one FP64 workgroup
+// fits a CU in place of two: 2^3 x 2^17 x 2^5 in complex FP64 179 us in place of
+// 127, real 75 of 52; only where whole lines of the long operand run along K does
+// it gain (2^3 x 2^17 x 2^7 157 to 110).
+constexpr int KSB = 2048;
 constexpr int KOFF_S = 2 * kSkinnyMaxK, KOFF_C = KOFF_S + kSkinnyMaxS, KOFF_N = KOFF_C + kSkinnyMaxS;
 
 // SM: the short side is M (A is the short operand, B the long one, C's long

@@ -255,7 +255,6 @@ constexpr int64_t kTickSingleMax = 256;
 // The power-of-two kernel's pairs (bits_pair; those of other extents keep the
 // shallow and skinny kernels).
 constexpr int64_t kBitMinTiles = 256, kBitSkinnyMaxK = 128, kBitSkinnyMinTiles = 512;
-constexpr int kBitSmallChunks = 4;
 // Work list (the persistent items, largest K first, then the shallow pairs'
 // items), workgroup count and LDS size of the pairs in lw.
 void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw);

@@ -87,21 +87,37 @@ void copy_desc(Batch& b, const muscle_hip_tensor_t& t, std::vector<muscle_hip_te
   dst.push_back(t);
 }
 
-// Shallow or skinny pairs that the power-of-two kernel is for (complex FP64, us):
-// the 256 pairs of a circuit network to rank 22, all by the other two kernels
-// 5213, by this one 4138, and 4215 where pairs of fewer than 128 of its tiles
-// stay with them (a launch of their own).  Where every pair is small they stay:
-// a server's ticks (up to 64 tiles a pair) ran this kernel for 52 us, of which
-// most is fetching its code and descriptors once, the others for 12 and 20.
-// A longer K is a chain of gathers: 2^3 x 2^8 x 2^7 (x 4) on its 4 tiles took
-// 60 us longer than the skinny kernel when its operands were in HBM, so from
-// 512 tiles on, as for a single contraction; and a small pair's K in at most 4
-// chunks (60 pairs to rank 20: 1232 us without this, 1161 with it, as by the
-// other kernels alone).
+// Shallow or skinny pairs that the power-of-two kernel is for, by size (complex
+// FP64, us): the 256 pairs of a circuit network to rank 22 take 5310 by the other
+// two kernels, 3800 with this one, and 2 % more where pairs of fewer than 128 of
+// its tiles stay with them (a launch of their own).  Where every pair is small
+// they stay: a server's ticks (up to 64 tiles a pair) ran this kernel for 52 us, of
+// which most is fetching its code and descriptors once, the others for 12 and 20.
+// K > 16 from 512 tiles on: 2^3 x 2^8 x 2^7 (x 4) on its 4 tiles took 60 us longer.
 bool bits_pair(const ContractionDesc& d, bool others) {
   const double tiles = (double)d.M * (double)d.N * (double)d.B / (1 << kBitTile);
   if (d.K <= kShallowK) return others || tiles >= kBitMinTiles;
   return std::min(d.M, d.N) <= kSkinnyMaxS && d.K <= kBitSkinnyMaxK && tiles >= kBitSkinnyMinTiles;
+}
+// And by plan.  Each K chunk is a round trip to memory that the skinny kernel
+// hides better, so the chunks decide (time over the other kernel's, 5764 launches
+// of one to four pairs, all four types, least / median / most): short side with
+// 1 or 2 chunks 0.26 / 0.62 / 1.02; 4 chunks and sides of 1 or 2 complex FP64 up to
+// 1.17, other types 0.57 / 0.85 / 1.11 unless a run of the long operand along its
+// rows is shorter than a line (1.0 to 2.5: a chunk fetches part of every line); 8 to
+// 32 chunks 0.5 to 2.0.  But where whole lines run along K the skinny kernel holds
+// them all between one k and the next: 0.32 / 0.65 / 1.04 from a side of 4 on (2 for
+// 4- and 8-byte types) with any number of chunks.  A side of 16 does four times the
+// work per element gathered: complex FP64 to 16 chunks 0.49 / 0.70 / 1.05, 8-byte
+// types to 8 0.45 / 0.8 / 1.24.  Both sides 32 or more, against the shallow kernel: 1
+// chunk 0.18 / 0.9 / 1.16; 2 in FP64 0.7 / 0.95 / 1.2, in FP32 0.9 / 1.05 / 1.2; 4
+// (K = 16) 1.0 to 1.9, but of 4096 or more complex FP64 tiles half.
+bool bits_pays(const ContractionDesc& d, const BitDesc& q) {
+  const int64_t side = std::min(d.M, d.N), es = (int64_t)dtype_size(d.dt[2]);
+  if (side > kSkinnyMaxS) return q.nchunk <= (es == 16 && q.tiles >= 4096 ? 4 : is_double(d.dt[2]) ? 2 : 1);
+  if (q.nchunk <= 2 || ((es << q.line_k) == 128 && side >= (es == 16 ? 4 : 2))) return true;
+  if (side == 16) return q.nchunk <= (es == 16 ? 16 : es == 8 ? 8 : 2);
+  return q.nchunk <= 4 && (es == 16 ? side == 8 : side * (128 >> q.line_k) > 32);
 }
 
 }  // namespace
@@ -134,7 +150,7 @@ void plan_pair(const Handle& h, PlannedPair& L, std::vector<int64_t>& htab, int 
   const int64_t lim = int64_t(1) << 31;
   if (d.M >= lim || d.N >= lim || d.K >= lim || d.B >= lim)
     fail(MUSCLE_HIP_UNSUPPORTED, "batched pair with an index class of 2^31 or more elements");
-  L.bits = bits_pair(d, false) && plan_bits(d, L.bit);
+  L.bits = bits_pair(d, false) && plan_bits(d, L.bit) && bits_pays(d, L.bit);
   L.bits_only = L.bits && d.K <= kShallowK;
   const std::vector<Dim>* cls[4] = {&d.m, &d.n, &d.k, &d.batch};
   for (int t = 0; t < 9 && !L.bits_only; ++t) L.t[t] = add_table(htab, *cls[T3[t][0]], T3[t][1], single_max);
@@ -278,8 +294,8 @@ void finish_batch(Handle& h, Batch& B, const std::vector<const PlannedPair*>& lw
         for (int64_t t = 0; t < items; ++t) xq[x].push_back(make_int2((int)i, (int)t));
         xload[x] += cost * (double)items;
       }
-    } else if ((sh || sk) && (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small) &&
-                                         small.nchunk <= kBitSmallChunks))) {
+    } else if ((sh || sk) &&
+               (L.bits || (run_bits && bits_pair(L.d, true) && plan_bits(L.d, small) && bits_pays(L.d, small)))) {
       const int32_t x = (int32_t)B.hbits.size();
       B.bit_index[(size_t)i] = x;
       B.hbits.push_back(L.bits ? L.bit : small);

@@ -31,6 +31,8 @@ struct BitDesc {
   int32_t tiles;
   int32_t kc, nchunk;  // K elements per chunk, chunks
   int32_t c_stream;
+  int32_t line_k;      // (host) bits of K inside a 128-byte line of the long operand,
+  int32_t line_split;  // and whether some of them belong to another chunk
   int32_t nl, ns;                // elements of a K chunk in the long and short operands (powers of two)
   int32_t sl, ss;                // LDS elements per k of each
   int32_t kxl, kxs;              // k bits folded into the low LDS bits of each

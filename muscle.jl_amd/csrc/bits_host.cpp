@@ -184,6 +184,11 @@ bool plan_bits(const ContractionDesc& d, BitDesc& out) {
   }
   out.kc = 1 << kcb;
   out.nchunk = 1 << (nk - kcb);
+  for (int j = 0; j < nk; ++j)
+    if (k[(size_t)j].s[lw] * es < 128) {
+      ++out.line_k;
+      if (j >= kcb) out.line_split = 1;
+    }
   uint32_t cl = 0, cs = 0;  // the lower bits' strides together
   for (int j = kcb; j < nk; ++j) {
     const uint32_t x = (uint32_t)k[(size_t)j].s[lw], y = (uint32_t)k[(size_t)j].s[sw];

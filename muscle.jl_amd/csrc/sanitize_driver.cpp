@@ -25,6 +25,7 @@
 #include <random>
 #include <vector>
 
+#include "batch.hpp"
 #include "handle.hpp"
 #include "muscle_hip.h"
 
@@ -554,6 +555,74 @@ void check_bits_empty() {
   expect(others > 0, "the same sizes with elements to sum", others);
 }
 
+// Which contractions the power-of-two kernel takes, plain and in a batch, on
+// both sides of the rules' lines: sides of 2^s and 2^n, K of 2^k, modes of two.
+// The long operand's lines run along its rows, or along K (kfast), or along
+// both (half of a line each); C has the short side's modes first.
+void check_bits_rules() {
+  enum Lines { ROWS, KFAST, HALF };
+  const int F32 = MUSCLE_HIP_F32, F64 = MUSCLE_HIP_F64, C32 = MUSCLE_HIP_C32, C64 = MUSCLE_HIP_C64;
+  struct {
+    int dt, s, n, k;
+    Lines lines;
+    bool plain, batch;
+  } rows[] = {
+      // one and two chunks, by tiles
+      {C64, 4, 14, 2, ROWS, true, false}, {C64, 4, 13, 2, ROWS, false, false}, {C64, 4, 15, 2, ROWS, true, true},
+      {F32, 3, 15, 3, ROWS, false, false}, {F32, 3, 16, 3, ROWS, true, true}, {F64, 2, 17, 4, ROWS, false, true},
+      // a short side and K in many chunks
+      {C64, 2, 18, 7, ROWS, true, false}, {C64, 2, 18, 7, KFAST, true, true}, {C64, 1, 19, 6, KFAST, false, false},
+      {C64, 0, 18, 3, HALF, false, false}, {C64, 0, 20, 3, ROWS, true, false}, {C64, 4, 16, 7, ROWS, true, true},
+      {F64, 2, 18, 7, ROWS, true, false}, {F64, 2, 18, 7, HALF, false, false}, {F64, 2, 18, 7, KFAST, true, true},
+      {F64, 0, 20, 3, HALF, false, false}, {F64, 0, 20, 3, KFAST, false, false}, {F64, 4, 16, 7, ROWS, false, false},
+      {C32, 1, 19, 5, KFAST, false, true}, {C32, 3, 17, 6, HALF, false, false}, {C32, 3, 18, 6, HALF, true, false},
+      {F32, 3, 18, 6, HALF, false, false}, {F32, 4, 16, 5, ROWS, false, false}, {F32, 4, 16, 6, KFAST, false, true},
+      {F32, 1, 19, 5, ROWS, true, false}, {F32, 1, 19, 5, HALF, false, false},
+      // K beyond 128, both sides long
+      {C64, 3, 17, 8, KFAST, false, false}, {C64, 5, 15, 5, ROWS, false, false}, {C64, 5, 6, 3, ROWS, true, false},
+      {F32, 5, 15, 4, ROWS, true, true}, {F64, 5, 17, 4, ROWS, false, true},
+  };
+  mh::Handle h;
+  int i = 0;
+  for (const auto& r : rows) {
+    Operand a, b, c;
+    auto put = [](Operand& o, int from, int count) {
+      for (int j = 0; j < count; ++j) {
+        o.strides.push_back(int64_t(1) << o.modes.size());
+        o.modes.push_back(from + j);
+        o.ext.push_back(2);
+      }
+    };
+    const int S = 1, N = S + r.s, K = N + r.n;
+    int line = 0;  // log2 of the elements of a line
+    while ((int64_t)esize(r.dt) << line < 128) ++line;
+    put(a, S, r.s);
+    put(a, K, r.k);
+    const int first = r.lines == ROWS ? 0 : r.lines == KFAST ? r.k : std::min(r.k, line - 1);
+    put(b, K, first);
+    put(b, N, r.n);
+    put(b, K + first, r.k - first);
+    put(c, S, r.s);
+    put(c, N, r.n);
+    const mh::ContractionDesc d =
+        mh::lower_binary(c.desc(r.dt, (void*)256), a.desc(r.dt, (void*)256), b.desc(r.dt, (void*)256));
+    mh::BitDesc q;
+    expect(mh::plan_bits(d, q), "power-of-two rule: the kernel could take it", i);
+    const bool plain = mh::build_contraction_plan(d, MUSCLE_HIP_PRECISION_NATIVE)->kind == mh::Plan::BITS;
+    mh::PlannedPair pair;
+    std::vector<int64_t> tab;
+    pair.d = d;
+    mh::plan_pair(h, pair, tab, MUSCLE_HIP_TILE_AUTO, mh::kTickSingleMax);
+    if (plain != r.plain || pair.bits != r.batch)
+      std::fprintf(stderr, "row %d: %d chunks, %d K bits in a line, %d tiles: plain %d, batch %d\n", i, q.nchunk, q.line_k,
+                   q.tiles, plain, pair.bits);
+    expect(plain == r.plain, "power-of-two rule: plain contraction", i);
+    expect(pair.bits == r.batch, "power-of-two rule: batched pair", i);
+    ++i;
+  }
+  std::printf("power-of-two kernel: %d contractions on both sides of its rules\n", i);
+}
+
 bool is_cplx(int dt) { return dt == MUSCLE_HIP_C32 || dt == MUSCLE_HIP_C64; }
 
 std::vector<char> encode(const std::vector<cd>& v, int dt) {
@@ -810,6 +879,7 @@ int main(int argc, char** argv) {
   std::mt19937_64 rng_o(20261205);
   check_bits_offsets(rng_o);
   check_bits_empty();
+  check_bits_rules();
   if (argc > 1 && std::strcmp(argv[1], "--gpu") == 0) check_gpu(rng);
   std::printf("%s: %d failures\n", g_failures ? "FAILED" : "ok", g_failures);
   return g_failures ? 1 : 0;
