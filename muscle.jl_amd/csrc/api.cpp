@@ -198,8 +198,6 @@ KTiles k_tiles(const ContractionDesc& d) {
   return r;
 }
 
-namespace {
-
 void plan_gemm_ktiles(Plan& p) {
   if (p.kind != Plan::GEMM) return;
   const KTiles t = k_tiles(p.d);
@@ -208,6 +206,8 @@ void plan_gemm_ktiles(Plan& p) {
   p.min_a = t.min_a;
   p.min_b = t.min_b;
 }
+
+namespace {
 
 // The contraction runs in its operands' own precision (no ladder rung).
 bool precision_plain(const ContractionDesc& d, int precision) {

@@ -131,6 +131,8 @@ struct KTiles {
   int64_t min_a, min_b;
 };
 KTiles k_tiles(const ContractionDesc& d);
+// The same for a tile-GEMM plan (plans of other kinds keep none).
+void plan_gemm_ktiles(Plan& p);
 void upload_tables(Plan& p, hipStream_t s);
 // Enqueues one planned contraction on h.stream.  Its workspace is the
 // handle's (grown as needed), or `ws` of `ws_size` bytes when given (no

@@ -28,6 +28,7 @@
 #include "batch.hpp"
 #include "handle.hpp"
 #include "muscle_hip.h"
+#include "split.hpp"
 
 namespace {
 
@@ -265,6 +266,22 @@ void check_ktiles(std::mt19937_64& rng) {
   }
   expect(set > plans / 2, "most plans have a common base per K-tile", set);
   std::printf("%lld tile GEMM plans checked, %lld K-tile sizes with a common base\n", (long long)plans, (long long)set);
+}
+
+// The FP32 rung's plan (FP64 operands rounded as they are gathered) has the
+// addressing of the plain plan on the same operands.
+void check_fp32_ktiles() {
+  for (int64_t k : {48, 512, 1728})
+    for (int dt : {MUSCLE_HIP_F64, MUSCLE_HIP_C64}) {
+      Operand a{{1, 2}, {300, k}, {1, 300}}, b{{2, 3}, {k, 500}, {1, k}}, c{{1, 3}, {300, 500}, {1, 300}};
+      const mh::ContractionDesc d = mh::lower_binary(c.desc(dt, (void*)256), a.desc(dt, (void*)256), b.desc(dt, (void*)256));
+      const std::unique_ptr<mh::Plan> p = mh::build_contraction_plan(d, MUSCLE_HIP_PRECISION_NATIVE);
+      const std::unique_ptr<mh::Plan> q = mh::build_contraction_plan(d, MUSCLE_HIP_PRECISION_FP32);
+      mh::prepare_split(*q, 1e-6);
+      expect(q->kind == mh::Plan::GEMM && q->fp32_math, "FP32 rung: plan", k);
+      expect(p->ktile8 && p->ktile16 && q->ktile8 && q->ktile16, "FP32 rung: common base per K-tile", k);
+      expect(p->min_a == q->min_a && p->min_b == q->min_b && p->gemm_kchunk == q->gemm_kchunk, "FP32 rung: base", k);
+    }
 }
 
 // The power-of-two kernel's plan, run on the host index by index as the kernel
@@ -875,6 +892,7 @@ int main(int argc, char** argv) {
   check_describe(rng);
   std::mt19937_64 rng_k(20261204);
   check_ktiles(rng_k);
+  check_fp32_ktiles();
   check_bits(rng_k);
   std::mt19937_64 rng_o(20261205);
   check_bits_offsets(rng_o);

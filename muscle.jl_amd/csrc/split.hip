@@ -739,6 +739,7 @@ void prepare_split(Plan& p, double target) {
     p.fp32_math = true;
     p.err_bound = fp32_model(d.K);
     plan_gemm_ksplit(p);
+    plan_gemm_ktiles(p);
     return;
   }
   const bool ca = is_complex(d.dt[0]), cb = is_complex(d.dt[1]);
