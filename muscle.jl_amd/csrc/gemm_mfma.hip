@@ -119,7 +119,6 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
   static_assert(NEA >= 1 && NEB >= 1 && BM + BN <= NT, "tile shape");
   static_assert(2 * (SA + SB) * sizeof(T) >= (BM + BN) * sizeof(int64_t), "C's offsets reuse the stages");
   __shared__ __attribute__((aligned(16))) T lds[2 * (SA + SB)];  // two A stages, then two B stages
-  __shared__ int64_t koff[SEP ? 1 : 2][2][BK];  // not SEP: byte offsets in A and B of a K-tile's k
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -172,6 +171,16 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
     }
   }
   auto at = [&](uint32_t off, int e) -> T& { return *((T*)((char*)lds + off) + e); };
+  // not SEP: byte offsets in A (w = 0) and B of k of the K-tile in buffer b; in
+  // FP64 in the padding of A's first rows (an array of its own left real FP64
+  // 64x64x16 three workgroups per CU in place of four: 2048 x 2048 x 510 143 us
+  // in place of 119)
+  constexpr bool KPAD = sizeof(T) == 8;
+  static_assert(BK <= LDP, "K offsets of one buffer and operand lie in one row's padding");
+  __shared__ int64_t ktab[SEP || KPAD ? 1 : 4 * BK];
+  auto koff = [&](int b, int w, int k) -> int64_t& {
+    return KPAD ? ((int64_t*)lds)[(2 * b + w) * LA + BM + k] : ktab[(2 * b + w) * BK + k];
+  };
 
   // K offsets of K-tile t (the last one's missing k clamped)
   auto k_offsets = [&](int t, int64_t* ka, int64_t* kb) {
@@ -237,7 +246,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
       for (int i = 0; i < NEA; ++i) pa[i] = (const char*)p.A + (offA0 + om[i]) * EA;
 #pragma unroll
       for (int i = 0; i < NEB; ++i) pb[i] = (const char*)p.B + (offB0 + on[i]) * EB;
-      if (tid < 2 * BK && nk > 1) koff[1][tid / BK][tid % BK] = k_entry(1);
+      if (tid < 2 * BK && nk > 1) koff(1, tid / BK, tid % BK) = k_entry(1);
     }
     if (nfull == 0) zero_tail();
   }
@@ -257,9 +266,9 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < NEA; ++i) ra[i] = load_elem<S, CA>(pa[i] + koff[t & 1][0][a_k(i)], 0);
+      for (int i = 0; i < NEA; ++i) ra[i] = load_elem<S, CA>(pa[i] + koff(t & 1, 0, a_k(i)), 0);
 #pragma unroll
-      for (int i = 0; i < NEB; ++i) rb[i] = load_elem<S, CB>(pb[i] + koff[t & 1][1][b_k(i)], 0);
+      for (int i = 0; i < NEB; ++i) rb[i] = load_elem<S, CB>(pb[i] + koff(t & 1, 1, b_k(i)), 0);
     }
   };
   auto gather_tail = [&]() {  // the last K-tile, of fewer than BK k
@@ -393,7 +402,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
       if (!inner && t + 1 == nfull) zero_tail();
       stash(cur ^ 1);
       if constexpr (!SEP)
-        if (tid < 2 * BK && t + 2 < nk) koff[cur][tid / BK][tid % BK] = kn;
+        if (tid < 2 * BK && t + 2 < nk) koff(cur, tid / BK, tid % BK) = kn;
     }
     __syncthreads();
   };
@@ -504,19 +513,33 @@ void launch_tile(GemmArgs g, hipStream_t s) {
 //   complex FP64, 64x64x8 / 32x64x8 / 32x32x8: N = 1024: 80 / 66 / 58, 1536:
 //     143 / 129 / 122, 2048: 231 / 203 / 213, 4096: 729 / 766 / 795;
 //     4096 x 4096 with K = 8 / 32 / 128: 52 / 82 / 209 against 47 / 82 / 219
-//     for 32x64x8; K = 4096: 5.69 ms, 5.59 with 64x64x16 (78 KB more LDS, two
-//     workgroups per CU in place of three, half the barriers);
+//     for 32x64x8; K = 4096: 5.69 ms, 5.59 with 64x64x16 (80 KB of LDS in place of
+//     40, two workgroups per CU in place of three, half the barriers);
 //   real FP64, 64x64x16 / 32x32x16: 1024: 32 / 26, 1536: 58 / 52, 2048: 75 / 88;
 //   ComplexF32, 64x64x8 / 32x64x16: 1024: 46 / 34, 1536: 75 / 76, 2048: 101 / 110;
-//     where K's modes leave no common base per K-tile (a lookup per k, fewer of
-//     them in a longer K-tile), 64x64x16 / 32x64x16: 1728 x 1728 x 1728 (729 tiles)
-//     339 / 377, and against 64x64x8 2197 x 2197 x 2197 710 / 801, but with K
-//     sliced (1000 x 1000 x 2197) 187 / 162;
 //   real FP32, 64x64x16 / 32x64x16: 1024: 22 / 17, 1536: 35 / 30, 2048: 43 / 49.
+// K of at most 32 is one or two K-tiles, and a wave of stores per tile: real FP64
+//   900 x 1900 x 16 8.8 / 10.0, 1200 x 2500 x 16 10.7 / 12.8, real FP32 the latter
+//   9.0 / 10.6, ComplexF32 12.5 / 13.8; with a side below 64, which every tile pads,
+//   real FP64 40000 x 2 x 24 10.8 / 7.9, FP32 131072 x 2 x 24 20.4 / 15.8.
+// Where K's modes leave no common base per K-tile (lookups), a tile costs a
+// chain of table reads before its first product:
+//   slices of at most 64 k: 512 x 512 x 510 real FP64 22.8 / 27.5, FP32 16.9 / 22.1,
+//     ComplexF32 25.7 / 29.5 (the FP32 rung's complex tiles 30.3 / 28.4), but real FP64 20 x
+//     4000 x 500 22.5 / 19.4;
+//   real FP64 from 640 tiles: 1900 x 1900 x 510 104 / 130;
+//   three workgroups per CU take 768 tiles: ComplexF32 64x64x16 / 32x64x16 1024 x
+//     3000 x 252 (768 tiles) 78 / 86, 1728 x 1728 x 1728 (729) 339 / 377, but 2048 x 2048
+//     x 126 (1024) 73 / 65, 2197 x 2197 x 2197 710 / 801 (64x64x8 in its place); real x
+//     complex FP64 2048 x 2048 x 126 78 / 73, 2300 x 2300 x 510 (1296) 245 / 260;
+//     with K sliced ComplexF32 1000 x 1000 x 2197 187 / 162.
 template <typename T, typename S, bool CA, bool CB, bool G3>
 void launch_t(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch * g.ksplit;
   const int k = std::min(g.K, g.kchunk);
+  const bool lookups = !((CA || CB) ? g.ktile8 : g.ktile16), wide = g.M >= 64 && g.N >= 64;
+  const bool shortk = k <= 32;
+  const bool brief = lookups && wide && g.ksplit > 1 && k <= 64 && tiles >= 256;
   if constexpr (sizeof(T) == 8 && CA && CB) {
     if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 8, 2, 2, 6, 1>>(g, s);
     else if (tiles < 2048 || k <= 32) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 1>>(g, s);
@@ -524,19 +547,21 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, G3 ? 3 : 2, 1>>(g, s);
   } else if constexpr (sizeof(T) == 8) {
     if constexpr (CA || CB) {
-      if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 2>>(g, s);
+      if (tiles < (lookups ? 1025 : 1024) && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 2>>(g, s);
       else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, 3, 1>>(g, s);
     } else {
-      if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 16, 2, 2, 6, 4>>(g, s);
+      if (shortk ? !wide || tiles < 400 : tiles < (lookups && wide ? 640 : 1024) && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 16, 2, 2, 6, 4>>(g, s);
       else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 4, 1>>(g, s);
     }
   } else if constexpr (CA || CB) {
-    const bool lookups = !g.ktile8 && g.ksplit == 1;
-    if (tiles < (lookups ? 640 : 1024)) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
-    else if (lookups) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 3, 1>>(g, s);
+    const bool whole = lookups && g.ksplit == 1;
+    const bool small = whole ? tiles < 640 || (tiles > 768 && tiles <= 1024)
+                             : tiles < (shortk && wide ? 640 : lookups && sizeof(S) == 8 ? 1025 : 1024) && !(brief && sizeof(S) == 4);
+    if (small) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
+    else if (whole) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 3, 1>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, sizeof(S) == 8 ? 3 : 4, 1>>(g, s);
   } else {
-    if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
+    if (shortk ? !wide || tiles < 400 : tiles < 1024 && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, sizeof(S) == 8 ? 3 : 4, 4>>(g, s);
   }
   if (g.ksplit > 1) {
