@@ -179,7 +179,7 @@ KTiles k_tiles(const ContractionDesc& d) {
   for (int w = 0; w < 2; ++w) {
     int64_t lo, hi, klo = 0, khi = 0;
     offset_range(w == 0 ? d.m : d.n, w, lo, hi);
-    std::vector<Dim> head, rest;
+    std::vector<Dim> head;
     int64_t n = 1;
     for (auto& x : d.k) {
       if (n >= 16) break;

@@ -101,8 +101,7 @@ __device__ __forceinline__ constexpr int swz(int k) {
 // SEP: the offset of every k is that of its K-tile's first k plus that of its
 // place in the tile, and a tile's elements span less than 2^32 bytes; else
 // K offsets of every K-tile are looked up one K-tile ahead, into LDS.
-// STEPS: MFMA steps (4 k each) whose operands are read and summed together; 0:
-// one at a time, the next step's reads issued ahead of the MFMAs.
+// STEPS: MFMA steps (4 k each) whose operands are read and summed together.
 template <typename T, typename S, bool CA, bool CB, bool G3, bool SEP, int BM, int BN, int BK, int WM, int WN, int OCC, int STEPS>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p) {
   using M_ = Mfma<T>;
@@ -369,34 +368,18 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(GemmArgs p
     int64_t kn = 0;  // K-tile t + 2's offsets replace K-tile t's
     if constexpr (!SEP)
       if (tid < 2 * BK && t + 2 < nk) kn = k_entry(t + 2);
-    if constexpr (STEPS == 0) {
-      // step by step, the next step's reads ahead of this step's MFMAs
-      Frag f[2];
-      read_frag(cur, 0, f[0]);
+    Frag f[STEPS];
+#pragma unroll
+    for (int k0 = 0; k0 < KS; k0 += STEPS) {
+#pragma unroll
+      for (int e = 0; e < STEPS; ++e) read_frag(cur, k0 + e, f[e]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        sums(f[ks & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (ks + 1 < KS) read_frag(cur, ks + 1, f[(ks + 1) & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(f[ks & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      Frag f[STEPS];
+      for (int e = 0; e < STEPS; ++e) sums(f[e]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k0 = 0; k0 < KS; k0 += STEPS) {
-#pragma unroll
-        for (int e = 0; e < STEPS; ++e) read_frag(cur, k0 + e, f[e]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int e = 0; e < STEPS; ++e) sums(f[e]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int e = 0; e < STEPS; ++e) multiply(f[e]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      for (int e = 0; e < STEPS; ++e) multiply(f[e]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     if (inner || t + 1 < nk) {
       if (!inner && t + 1 == nfull) zero_tail();
@@ -484,25 +467,21 @@ __global__ __launch_bounds__(NTF) void splitk_finish_kernel(GemmArgs p) {
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int OCC_, int STEPS_>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, OCC = OCC_, STEPS = STEPS_;
-  // complex FP64 64x64x16 fills the LDS of two workgroups per CU: no room for the K offset table
-  static constexpr bool SEP_ONLY = BM == 64 && BN == 64 && BK == 16 && OCC == 2;
 };
 
-template <typename T, typename S, bool CA, bool CB, bool G3, typename C>
-void launch_tile(GemmArgs g, hipStream_t s) {
+// SEP: this kernel of the configuration (a common base per K-tile, or lookups).
+template <typename T, typename S, bool CA, bool CB, bool G3, bool SEP, typename C>
+void launch_kernel(GemmArgs g, hipStream_t s) {
   g.tiles_m = (g.M + C::BM - 1) / C::BM;
   g.tiles_n = (g.N + C::BN - 1) / C::BN;
   const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)g.batch, (unsigned)g.ksplit), block(64 * C::WM * C::WN);
-  if (C::BK == 8 ? g.ktile8 : g.ktile16)
-    hipLaunchKernelGGL(
-        (gemm_tile_kernel<T, S, CA, CB, G3, true, C::BM, C::BN, C::BK, C::WM, C::WN, C::OCC, C::STEPS>), grid, block, 0,
-        s, g);
-  else if constexpr (C::SEP_ONLY)
-    ;  // chosen for its K-tiles' common base only
-  else
-    hipLaunchKernelGGL(
-        (gemm_tile_kernel<T, S, CA, CB, G3, false, C::BM, C::BN, C::BK, C::WM, C::WN, C::OCC, C::STEPS>), grid, block,
-        0, s, g);
+  hipLaunchKernelGGL((gemm_tile_kernel<T, S, CA, CB, G3, SEP, C::BM, C::BN, C::BK, C::WM, C::WN, C::OCC, C::STEPS>), grid,
+                     block, 0, s, g);
+}
+template <typename T, typename S, bool CA, bool CB, bool G3, typename C>
+void launch_tile(const GemmArgs& g, hipStream_t s) {
+  if (C::BK == 8 ? g.ktile8 : g.ktile16) launch_kernel<T, S, CA, CB, G3, true, C>(g, s);
+  else launch_kernel<T, S, CA, CB, G3, false, C>(g, s);
 }
 
 // Tile shapes by the number of 64 x 64 tiles (and K slices) of the launch.
@@ -543,7 +522,7 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
   if constexpr (sizeof(T) == 8 && CA && CB) {
     if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 8, 2, 2, 6, 1>>(g, s);
     else if (tiles < 2048 || k <= 32) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 1>>(g, s);
-    else if (G3 && k >= 1024 && g.ktile16) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 2, 2>>(g, s);
+    else if (G3 && k >= 1024 && g.ktile16) launch_kernel<T, S, CA, CB, G3, true, Tile<64, 64, 16, 2, 2, 2, 2>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, G3 ? 3 : 2, 1>>(g, s);
   } else if constexpr (sizeof(T) == 8) {
     if constexpr (CA || CB) {
