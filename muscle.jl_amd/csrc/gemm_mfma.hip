@@ -499,8 +499,9 @@ void launch_tile(const GemmArgs& g, hipStream_t s) {
 //   real FP32, 64x64x16 / 32x64x16: 1024: 22 / 17, 1536: 35 / 30, 2048: 43 / 49.
 // K of at most 32 is one or two K-tiles, and a wave of stores per tile: real FP64
 //   900 x 1900 x 16 8.8 / 10.0, 1200 x 2500 x 16 10.7 / 12.8, real FP32 the latter
-//   9.0 / 10.6, ComplexF32 12.5 / 13.8; with a side below 64, which every tile pads,
-//   real FP64 40000 x 2 x 24 10.8 / 7.9, FP32 131072 x 2 x 24 20.4 / 15.8.
+//   9.0 / 10.6, ComplexF32 12.5 / 13.8; with a side below 64 and a last K-tile cut
+//   off (looked up again) FP64 40000 x 2 x 24 10.8 / 7.9, FP32 131072 x 2 x 24 20.4 /
+//   15.8, without FP32 65536 x 16 x 16 8.9 / 11.0.
 // Where K's modes leave no common base per K-tile (lookups), a tile costs a
 // chain of table reads before its first product:
 //   slices of at most 64 k: 512 x 512 x 510 real FP64 22.8 / 27.5, FP32 16.9 / 22.1,
@@ -517,7 +518,7 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
   const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch * g.ksplit;
   const int k = std::min(g.K, g.kchunk);
   const bool lookups = !((CA || CB) ? g.ktile8 : g.ktile16), wide = g.M >= 64 && g.N >= 64;
-  const bool shortk = k <= 32;
+  const bool shortk = k <= 32 && wide, thin_tail = k <= 32 && !wide && g.K % 16;
   const bool brief = lookups && wide && g.ksplit > 1 && k <= 64 && tiles >= 256;
   if constexpr (sizeof(T) == 8 && CA && CB) {
     if (tiles < 1024) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 8, 2, 2, 6, 1>>(g, s);
@@ -529,18 +530,18 @@ void launch_t(const GemmArgs& g, hipStream_t s) {
       if (tiles < (lookups ? 1025 : 1024) && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 8, 2, 2, 4, 2>>(g, s);
       else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, 3, 1>>(g, s);
     } else {
-      if (shortk ? !wide || tiles < 400 : tiles < (lookups && wide ? 640 : 1024) && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 16, 2, 2, 6, 4>>(g, s);
+      if (shortk ? tiles < 400 : thin_tail || (tiles < (lookups && wide ? 640 : 1024) && !brief)) launch_tile<T, S, CA, CB, G3, Tile<32, 32, 16, 2, 2, 6, 4>>(g, s);
       else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 4, 1>>(g, s);
     }
   } else if constexpr (CA || CB) {
     const bool whole = lookups && g.ksplit == 1;
     const bool small = whole ? tiles < 640 || (tiles > 768 && tiles <= 1024)
-                             : tiles < (shortk && wide ? 640 : lookups && sizeof(S) == 8 ? 1025 : 1024) && !(brief && sizeof(S) == 4);
+                             : tiles < (shortk ? 640 : lookups && sizeof(S) == 8 ? 1025 : 1024) && !(brief && sizeof(S) == 4);
     if (small) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 4, 1>>(g, s);
     else if (whole) launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, 3, 1>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 8, 2, 2, sizeof(S) == 8 ? 3 : 4, 1>>(g, s);
   } else {
-    if (shortk ? !wide || tiles < 400 : tiles < 1024 && !brief) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
+    if (shortk ? tiles < 400 : thin_tail || (tiles < 1024 && !brief)) launch_tile<T, S, CA, CB, G3, Tile<32, 64, 16, 2, 2, 5, 4>>(g, s);
     else launch_tile<T, S, CA, CB, G3, Tile<64, 64, 16, 2, 2, sizeof(S) == 8 ? 3 : 4, 4>>(g, s);
   }
   if (g.ksplit > 1) {
