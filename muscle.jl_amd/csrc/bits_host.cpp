@@ -123,6 +123,9 @@ bool plan_bits(const ContractionDesc& d, BitDesc& out) {
     if (c[(size_t)i].cls == scls) us.push_back(i);
   }
   const int rs = std::min<int>((int)us.size(), ul.size() >= 2 ? 1 : 2), rl = std::min<int>((int)ul.size(), kBitReg - rs);
+  // (not taken: C's six lowest bits all of one side and more than five of the
+  // other, such as the default output order where both sides are long; the
+  // tile then has no upper bit of the long operand for a register)
   if (rl + rs != kBitReg || rl == 0) return false;
   reg.assign(ul.end() - rl, ul.end());
   reg.insert(reg.end(), us.end() - rs, us.end());
