@@ -25,7 +25,10 @@
 // and 105; 2^12 x 2^12 x 2^2 86 and 76; 2^4 x 2^18 x 2^6 184 and 98; the
 // shallow and skinny pairs of a 256-pair batch (8.2 GB) 3.2 and 2.1 ms.  Bound
 // by memory; below some 100 tiles by fetching this code (8 KB a variant, run
-// once) and the descriptor, so small contractions stay with the others.
+// once) and the descriptor, so small contractions stay with the others, and by
+// the round trip of every K chunk, so most with many chunks do (bits_for,
+// bits_pays).  plan_bits leaves out what the tiles cannot hold: two long sides
+// in C's default order, a tile over 4 GiB, an empty sum.
 #include "bits.hpp"
 
 #include <algorithm>
